@@ -9,8 +9,8 @@ at 50 um / 150 mm, wavelength 0.2 A, omega 0-180 deg in 0.25 deg frames,
 timed region.  value = K*N*steps / elapsed.
 
 Printed: ONE JSON line, with a roofline object for the dominant kernel
-(k_score_many_sieve at tol <= 0.1, else k_score_many_fast; FP64 vector ALU
-bound) timed live with HIP events on its
+(k_score_mfma at tol <= 0.1, a sieve on the matrix cores; else
+k_score_many_fast, FP64 vector ALU bound) timed live with HIP events on its
 stream, and a cpu_baseline object: the reference C (oracle/_ref, compiled
 from its sources) running the same pipeline on the host cores, the grain
 loop spread over threads (ctypes releases the GIL), with its per-grain
@@ -36,19 +36,11 @@ ROOT = os.path.dirname(os.path.abspath(__file__))
 sys.path.insert(0, ROOT)
 
 FLOPS_PER_PAIR = 23      # h = UBI.g: 9 mul + 6 add; 3 sub; sumsq: 3 mul + 2 add
-# FP64 VALU instructions issued per pair by the certified kernel: rows
-# h + 1/2 with 3 FMA each (9), fract per row (3), sum f (f - 1) in 5, two
-# compares (2)
-VALU_OPS_PER_PAIR = 19
-# the sieved score (k_score_many_sieve<4>, the default for tol <= 0.1),
-# counted in its gfx950 assembly: every pair 8.5 VALU (row 0 + r by three
-# FMAs, v_fract_f64, one compare; two mbcnt and the queue address; one
-# entry per grain step for all four slots), every pair passing row 0
-# another 26.5 (17 FP64 of the certified test, the entry decode, addresses
-# and compares).  The SQ counters count 12.3 per pair in all, the tile
-# setup and the queue drains included.
-SIEVE_STAGE1_VALU = 8.5
-SIEVE_SETTLE_VALU = 26.5
+# the matrix-core sieve (k_score_mfma, the default for tol <= 0.1): three
+# v_mfma_f32_32x32x16_f16 for 32 peaks x 32 grains, i.e. 96 f16 flops per
+# pair executed (9 of the 16 k slots carry the split products)
+MFMA_FLOPS_PER_PAIR = 96
+PEAK_F16_MFMA = 2.5e15  # MI355X f16 matrix, dense
 # FP64 VALU instructions per pair of the fused compute_gv + score_and_assign
 # kernel's certified loop, counted in its gfx950 assembly: 70 per grain step
 # of two peaks per lane (22 v_fmac, 16 v_fma, 8 v_mul, 12 v_add, 6
@@ -918,20 +910,16 @@ def main():
     score_ms = statistics.mean(a.elapsed_time(b) for a, b in evs)
     pairs = args.grains * args.peaks
     value = pairs * args.steps / (total_ms * 1e-3)
-    achieved = FLOPS_PER_PAIR * pairs / (score_ms * 1e-3)
-    if batched.score_mode(args.tol) == _lib.SCORE_SIEVE:
-        kernel = "k_score_many_sieve"
-        g = batched.sf2gv(sc, fc, om, pars)
-        passed = 0.0
-        for k0 in range(0, min(args.grains, 64), 16):  # pairs passing row 0, 64 grains
-            h0 = ubis[k0:k0 + 16, 0, :] @ g.T
-            passed += float(((h0 - torch.round(h0)).abs() < args.tol).sum())
-            del h0
-        pass_frac = passed / (min(args.grains, 64) * args.peaks)
-        valu_ops = SIEVE_STAGE1_VALU + SIEVE_SETTLE_VALU * pass_frac
-        del g
+    if (batched.score_mode(args.tol) == _lib.SCORE_SIEVE and
+            batched.mfma_pays(args.grains, args.peaks)):
+        kernel, bound, peak = "k_score_mfma", "mfma", PEAK_F16_MFMA
+        achieved = MFMA_FLOPS_PER_PAIR * pairs / (score_ms * 1e-3)
+        frac_is = ("f16 matrix flops executed over the dense f16 peak; the kernel's vector "
+                   "instructions (3 per pair) run beside them, and the power limit bounds both")
     else:
-        kernel, pass_frac, valu_ops = "k_score_many_fast", None, VALU_OPS_PER_PAIR
+        kernel, bound, peak = "k_score_many_fast", "valu", PEAK_FP64_VALU
+        achieved = FLOPS_PER_PAIR * pairs / (score_ms * 1e-3)
+        frac_is = "algorithmic: flops_per_pair for every pair decided, over the FP64 peak"
     gpu_counts = counts.cpu().numpy()
     # boundary-peak audit of the device-sincos g-vectors (outside the timed
     # region): pairs within 1e-12 relative of tol^2, where a last-bit
@@ -970,21 +958,17 @@ def main():
                                "aux.refine_5000_grains.speedup_refine_plus_adjoint_vs_gpu_loop"},
         "roofline": {
             "kernel": kernel,
-            "bound": "valu",
+            "bound": bound,
             "achieved": achieved / 1e12,
-            "peak": PEAK_FP64_VALU / 1e12,
+            "peak": peak / 1e12,
             "unit": "TFLOP/s",
-            "frac": achieved / PEAK_FP64_VALU,
-            "frac_is": "algorithmic: flops_per_pair for every pair decided, over the FP64 "
-                       "peak; the kernel issues valu_ops_per_pair instructions per pair, "
-                       "and issued_valu_ops_frac_of_nonfma_peak is their issue rate",
+            "frac": achieved / peak,
+            "frac_is": frac_is,
             "traffic": measured_traffic(kernel),
             "kernel_ms": score_ms,
             "flops_per_pair": FLOPS_PER_PAIR,
-            "valu_ops_per_pair": valu_ops,
-            "row0_pass_fraction": pass_frac,
-            "issued_valu_ops_frac_of_nonfma_peak": valu_ops * pairs / (score_ms * 1e-3)
-            / (PEAK_FP64_VALU / 2),
+            "algorithmic_over_fp64_peak": FLOPS_PER_PAIR * pairs / (score_ms * 1e-3)
+            / PEAK_FP64_VALU,
         },
         "cpu_baseline": None,
     }

@@ -48,6 +48,8 @@ SIGNATURES = {
     "compute_gv": (None, [_vp, _vp, _d, _d, _d, _d, _vp, _vp, _i]),
     "compute_xlylzl": (None, [_vp, _vp, _vp, _vp, _vp, _vp, _i]),
     "gs_score_many": (_i, [_vp, _i, _vp, _i, _d, _vp, _i, _i, _vp]),
+    "gs_sieve_workspace_bytes": (ctypes.c_longlong, [_i]),
+    "gs_score_many_ws": (_i, [_vp, _i, _vp, _i, _d, _vp, _vp, _vp]),
     "gs_assign_many": (_i, [_vp, _vp, _i, _vp, _i, _d, _vp, _vp, _vp, _i, _vp]),
     "gs_score_and_refine_dev": (_i, [_vp, _vp, _i, _d, _vp, _vp, _vp]),
     "gs_refine_assigned_dev": (_i, [_vp, _vp, _i, _vp, _i, _vp, _vp, _vp]),
@@ -132,13 +134,13 @@ SIGNATURES = {
 SCORE_CERTIFIED = 0
 SCORE_EXACT = 1
 SCORE_SIEVE = 2
-SIEVE_TOL_MAX = 0.1  # the one-row sieve pays while ~2 tol of the pairs pass row 0
+SIEVE_TOL_MAX = 0.1  # the sieves pay while few of the pairs pass them
 
 
 def score_mode(tol):
-    """The faster of the certified score kernels for this tolerance: the
-    sieve (row 0 of every pair first) for |tol| <= SIEVE_TOL_MAX, else the
-    all-rows certified kernel.  Both give the reference's counts."""
+    """The faster kind of score kernel for this tolerance: a sieve for
+    |tol| <= SIEVE_TOL_MAX, else the all-rows certified kernel.  Both give
+    the reference's counts."""
     return SCORE_SIEVE if abs(float(tol)) <= SIEVE_TOL_MAX else SCORE_CERTIFIED
 
 _lib = None
@@ -230,6 +232,12 @@ def dptr(t):
 def hptr(a):
     """Host address of a numpy array's first element."""
     return ctypes.c_void_p(a.ctypes.data)
+
+
+def sieve_ws(K, device):
+    """Device workspace of the matrix-core sieve for K grains
+    (gs_sieve_workspace_bytes(K) bytes)."""
+    return torch.empty((K + 31) // 32 * 3088, dtype=torch.uint8, device=device)
 
 
 def darr(values):

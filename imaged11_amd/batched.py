@@ -38,13 +38,39 @@ def _ready():
 from ._lib import SIEVE_TOL_MAX, score_mode  # noqa: E402  (the default score kernel)
 
 
+def mfma_pays(K, N):
+    """Whether the matrix-core sieve is the faster one for K grains x N
+    peaks.  Its tiles hold 32 grains, and its workspace costs the host 1.4 us
+    a call: at 16 x 1e6 both sieves take 30 us, below 1e7 pairs both are
+    bound by the host (13.5 us against 14.9 at 300 x 10^4, 23.2 against 17.2
+    at 1000 x 3 10^4)."""
+    return K >= 24 and K * N >= 12000000
+
+
+def score_sieve(ubis, gv, tol, out=None):
+    """score_many by the sieve on the matrix cores (gs_score_many_ws), at any
+    size and tolerance."""
+    lib = _ready()
+    _need(ubis, torch.float64, "ubis", (None, 3, 3))
+    _need(gv, torch.float64, "gv", (None, 3))
+    K = ubis.shape[0]
+    if out is None:
+        out = torch.empty(K, dtype=torch.int32, device=gv.device)
+    _need(out, torch.int32, "out", (K,))
+    ws = _lib.sieve_ws(K, gv.device)
+    _lib.check(lib.gs_score_many_ws(dptr(ubis), K, dptr(gv), gv.shape[0], float(tol), dptr(out),
+                                    dptr(ws), stream_ptr()), "score_sieve")
+    return out
+
+
 def score_many(ubis, gv, tol, peaks_per_lane=0, out=None, exact=False, mode=None):
     """counts[g] = score(ubis[g], gv, tol) for every grain g.
 
     ubis (K,3,3) float64, gv (N,3) float64 -> int32 (K,).  exact=True uses
     the reference's arithmetic for every pair; by default the certified
     kernel score_mode(tol) picks runs; every mode returns the reference's
-    counts."""
+    counts.  Of the two sieves, mfma_pays(K, N) picks (a tile height
+    peaks_per_lane asks for the row sieve on the vector ALU)."""
     lib = _ready()
     _need(ubis, torch.float64, "ubis", (None, 3, 3))
     _need(gv, torch.float64, "gv", (None, 3))
@@ -54,6 +80,8 @@ def score_many(ubis, gv, tol, peaks_per_lane=0, out=None, exact=False, mode=None
     _need(out, torch.int32, "out", (K,))
     if mode is None:
         mode = _lib.SCORE_EXACT if exact else score_mode(tol)
+    if mode == _lib.SCORE_SIEVE and not peaks_per_lane and mfma_pays(K, gv.shape[0]):
+        return score_sieve(ubis, gv, tol, out)
     _lib.check(lib.gs_score_many(dptr(ubis), K, dptr(gv), gv.shape[0], float(tol), dptr(out),
                                  int(peaks_per_lane), mode, stream_ptr()), "score_many")
     return out

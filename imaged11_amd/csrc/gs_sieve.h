@@ -1,0 +1,346 @@
+// Sieve on the matrix cores for the all-pairs kernels.
+//
+// Whether |h_i - round(h_i)| < tol for the three rows h = UBI.g needs h only
+// to a small fraction of tol, and only modulo 1.  v_mfma_f32_32x32x16_f16
+// gives 32 peaks x 32 grains of one row from 16 products each, and with the
+// f32 accumulator started at 1.5 2^23 its last bit is worth exactly 1.  With
+// every product scaled by 2^16 the low 16 bits of the accumulator's own bit
+// pattern are then the fraction of h in units of 2^-16: no subtraction,
+// rounding or conversion is left for the vector ALU, which takes the maximum
+// of three 16-bit fields, the minimum over four pairs, and compares that:
+// three 16-bit instructions (2.4-2.8 cycles per wave each; v_max3_u16 and
+// v_min3_u16 take 8.4) and a quarter of a compare (4.2) per pair, against 11
+// FP64 instructions (4.5) of the row sieve k_score_many_sieve.  The MFMA's 32
+// cycles per 1024 products overlap them.  Measured, 1000 grains x 10^6 peaks,
+// tol 0.05: 146 us against 386; with the queue pushes off 120, with the
+// settling off 128.  What bounds it is the power limit: the same loop over
+// zeros runs a third faster than over data (201 against 270 cycles per tile).
+//
+// Splitting.  u and g are each held as hi + lo in f16 (22 bits), and the
+// products hi hi + hi lo + lo hi use 9 of the 16 k slots:
+//   k      0..2      3..5      6..8      9..15
+//   peak   gh_j      gl_j      gh_j      p_0..p_6
+//   grain  uh_j      uh_j      ul_j      q_0..q_6
+// with u' = 2^6 u and g' = 2^10 g (so that the low parts are normal f16
+// numbers) and p, q free for terms that depend on the grain's position.
+//
+// Certification.  With |u| < 900 and |g| < 30 (no overflow of f16) and
+// A = sum_j |u_ij| max|g_j| <= GS_SIEVE_SPAN for every row:
+//   hi + lo is within 2^-22 of u' (g') relative, or 2^-25 absolute where lo
+//   is subnormal, the product lo lo that is left out is below 2^-22 |u' g'|:
+//   together < 3 2^-22 A + 2^-31 (|u|_1 + |g|_1) 2^5 < 5e-5;
+//   the products of two f16 numbers are exact in f32, and each of the 17
+//   additions, of whatever order and of rounding or truncation, keeps the
+//   accumulator in [2^23, 2^24) or below it and is therefore within one unit
+//   of its last place, 2^-16 of h: < 2.6e-4.
+// So h is within GS_SIEVE_ERR = 2^-11 = 4.9e-4, tested with r = tol + 2^-11
+// (+ the reference's own rounding of h and t, 1e-12): a pair with
+// fract(h + r) > 2r in any row has a reference drlv2 >= tol^2 and is not
+// counted.  The others (the cube of side 2r, 0.1% of random pairs at tol
+// 0.05, and the true hits) are settled one by one with the reference
+// arithmetic, so the sieve decides nothing that arithmetic would not.
+// A pair with a non-finite u or g has a NaN drlv2 and never counts: it may
+// pass or not, and is kept out of the bounds; peaks with one are given a
+// finite stand-in.  Larger A: up to GS_SIEVE_SPAN_WIDE the accumulator
+// starts at 1.5 2^27 (its last bit 2^-12 of h) and the fields are shifted
+// left by four first, error GS_SIEVE_ERR_WIDE = 2^-7 by the same count;
+// beyond that every pair takes the reference arithmetic.
+#pragma once
+#include "gs_kernels.h"
+
+typedef _Float16 gs_half8 __attribute__((ext_vector_type(8)));
+typedef float gs_float16 __attribute__((ext_vector_type(16)));
+
+#define GS_SIEVE_SPAN 60.0f
+#define GS_SIEVE_SPAN_WIDE 1000.0f
+#define GS_SIEVE_UMAX 900.0f
+#define GS_SIEVE_GMAX 30.0f
+#define GS_SIEVE_ERR 0x1p-11
+#define GS_SIEVE_ERR_WIDE 0x1p-7
+#define GS_SIEVE_SETS 4    // 32-peak sets per wave (NB)
+#define GS_SIEVE_SPLIT 64  // grain tiles of a block's split at most (its counters in LDS)
+
+// v = hi + lo in f16, for a scaled value below the f16 range
+GS_HD __forceinline__ void gs_split16(double v, _Float16& hi, _Float16& lo) {
+    hi = (_Float16)(float)v;
+    lo = (_Float16)(float)(v - (double)(float)hi);
+}
+
+// the sieve radius in units of 2^-16 (the threshold is twice it), 0x7fff
+// with threshold 0xffff (every pair passes) where 2r would reach 1
+GS_HD __forceinline__ void gs_sieve_units(double r, int& r16, int& thr) {
+    if (r < 0.49) {
+        r16 = (int)(r * 65536.0) + 2;
+        thr = 2 * r16;
+    } else {
+        r16 = 0;
+        thr = 0xffff;
+    }
+}
+
+// A peak's 16 k slots, the half this lane holds (k = 8 half + j); p may be
+// NULL (slots 9..15 zero)
+__device__ __forceinline__ gs_half8 gs_peak_frag(double g0, double g1, double g2, const double* p,
+                                                 int half) {
+    _Float16 h[3], l[3];
+    gs_split16(g0 * 1024.0, h[0], l[0]);
+    gs_split16(g1 * 1024.0, h[1], l[1]);
+    gs_split16(g2 * 1024.0, h[2], l[2]);
+    gs_half8 f;
+    f[0] = half ? h[2] : h[0];
+    f[1] = half ? (p ? (_Float16)(float)p[0] : (_Float16)0) : h[1];
+    f[2] = half ? (p ? (_Float16)(float)p[1] : (_Float16)0) : h[2];
+    f[3] = half ? (p ? (_Float16)(float)p[2] : (_Float16)0) : l[0];
+    f[4] = half ? (p ? (_Float16)(float)p[3] : (_Float16)0) : l[1];
+    f[5] = half ? (p ? (_Float16)(float)p[4] : (_Float16)0) : l[2];
+    f[6] = half ? (p ? (_Float16)(float)p[5] : (_Float16)0) : h[0];
+    f[7] = half ? (p ? (_Float16)(float)p[6] : (_Float16)0) : h[1];
+    return f;
+}
+
+// Both halves of a grain row's 16 k slots
+__device__ __forceinline__ void gs_grain_frag(double u0, double u1, double u2, const double* q,
+                                              gs_half8& a, gs_half8& b) {
+    _Float16 h[3], l[3];
+    gs_split16(u0 * 64.0, h[0], l[0]);
+    gs_split16(u1 * 64.0, h[1], l[1]);
+    gs_split16(u2 * 64.0, h[2], l[2]);
+    a = (gs_half8){h[0], h[1], h[2], h[0], h[1], h[2], l[0], l[1]};
+    b[0] = l[2];
+#pragma unroll
+    for (int i = 0; i < 7; i++) b[1 + i] = q ? (_Float16)(float)q[i] : (_Float16)0;
+}
+
+__device__ __forceinline__ bool gs_finite(double a) { return fabs(a) < __builtin_inf(); }
+
+// the 16-bit fraction fields of the three rows of one pair: the largest
+template <bool WIDE>
+__device__ __forceinline__ unsigned short gs_sieve_field(float a, float b, float c) {
+    unsigned short x = (unsigned short)__builtin_bit_cast(unsigned, a);
+    unsigned short y = (unsigned short)__builtin_bit_cast(unsigned, b);
+    unsigned short z = (unsigned short)__builtin_bit_cast(unsigned, c);
+    if (WIDE) {
+        x = (unsigned short)(x << 4);
+        y = (unsigned short)(y << 4);
+        z = (unsigned short)(z << 4);
+    }
+    unsigned short m = __builtin_elementwise_max(x, y);
+    // two v_max_u16 (2.4 cycles each), not one v_max3_u16 (8.4 cycles)
+    asm("" : "+v"(m));
+    return __builtin_elementwise_max(m, z);
+}
+
+// One 32-peak x 32-grain tile.  Accumulator register i of a lane holds peak
+// 8 (i / 4) + 4 (lane >> 5) + i % 4 and grain lane & 31, so registers 4 j ..
+// 4 j + 3 are four consecutive peaks against one grain: the smallest of their
+// four fields is compared (one compare and one branch for four pairs), and
+// where it passes the quad is appended to the wave's queue, entry lp + 2 j.
+// The queue's fill qn is wave-uniform; at most 256 entries are added, in
+// order of j, then lane.
+template <bool WIDE>
+__device__ __forceinline__ void gs_sieve_tile(gs_half8 pk, gs_half8 b0, gs_half8 b1, gs_half8 b2,
+                                              gs_float16 c, unsigned short thr, unsigned lp,
+                                              unsigned short* q, int& qn) {
+    const gs_float16 h0 = __builtin_amdgcn_mfma_f32_32x32x16_f16(pk, b0, c, 0, 0, 0);
+    const gs_float16 h1 = __builtin_amdgcn_mfma_f32_32x32x16_f16(pk, b1, c, 0, 0, 0);
+    const gs_float16 h2 = __builtin_amdgcn_mfma_f32_32x32x16_f16(pk, b2, c, 0, 0, 0);
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        unsigned short f = gs_sieve_field<WIDE>(h0[4 * j], h1[4 * j], h2[4 * j]);
+#pragma unroll
+        for (int i = 4 * j + 1; i < 4 * j + 4; i++) {
+            f = __builtin_elementwise_min(f, gs_sieve_field<WIDE>(h0[i], h1[i], h2[i]));
+            asm("" : "+v"(f));  // as in gs_sieve_field: no v_min3_u16
+        }
+        const bool in = f <= thr;
+        const unsigned long long m = __builtin_amdgcn_ballot_w64(in);
+        if (m) {
+            if (in) {
+                const unsigned pos = __builtin_amdgcn_mbcnt_hi(
+                    (unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u));
+                (q + qn)[pos] = (unsigned short)(lp + 2 * j);
+            }
+            qn += __popcll(m);
+        }
+    }
+}
+
+__device__ __forceinline__ gs_float16 gs_splat16(float v) {
+    return (gs_float16){v, v, v, v, v, v, v, v, v, v, v, v, v, v, v, v};
+}
+
+// ---------------------------------------------------------------------------
+// The grains' fragments, packed once per call into the caller's workspace:
+// tile t (grains 32 t .. 32 t + 31; past K the last grain again) has
+// 3 x 64 x 16 bytes, row-major by UBI row, lane l holding column l & 31 and k
+// slots 8 (l >> 5) .. + 7, then one float per tile, the largest row sum of
+// |u|.  Also clears counts (so that no separate fill is launched).
+inline long long gs_sieve_tiles(long long K) { return (K + 31) / 32; }
+inline long long gs_sieve_ws_bytes(long long K) { return gs_sieve_tiles(K) * (3 * 64 * 16 + 16); }
+
+__global__ __launch_bounds__(128) void k_sieve_pack(const double* __restrict__ ubis, int K,
+                                                    gs_half8* __restrict__ frag,
+                                                    float* __restrict__ span,
+                                                    int* __restrict__ counts) {
+    __shared__ float lspan[96];
+    const int tl = blockIdx.x, t = threadIdx.x;
+    if (t < 32 && 32 * tl + t < K) counts[32 * tl + t] = 0;
+    if (t < 96) {  // one grain row each
+        const int row = t / 32, col = t & 31;
+        const int g = min(32 * tl + col, K - 1);
+        const double* u = ubis + 9 * (size_t)g + 3 * row;
+        double u0 = u[0], u1 = u[1], u2 = u[2];
+        float a = (float)(fabs(u0) + fabs(u1) + fabs(u2));
+        if (!(a < __builtin_inff())) {  // never counted, whatever it passes
+            u0 = u1 = u2 = 0.0;
+            a = 0.0f;
+        }
+        lspan[t] = a * (1.0f + 0x1p-20f);
+        gs_half8* f = frag + (3 * (size_t)tl + row) * GS_WAVE;
+        gs_half8 lo, hi;
+        gs_grain_frag(u0, u1, u2, nullptr, lo, hi);
+        f[col] = lo;
+        f[col + 32] = hi;
+    }
+    __syncthreads();
+    if (t == 0) {
+        float a = lspan[0];
+        for (int i = 1; i < 96; i++) a = fmaxf(a, lspan[i]);
+        span[tl] = a;
+    }
+}
+
+// ---------------------------------------------------------------------------
+// score (and list extraction) for K UBIs x ng g-vectors.  A wave owns NB sets
+// of 32 peaks, their fragments in LDS, and goes through the block's split of
+// grain tiles, whose fragments it reads from the workspace one tile ahead.
+// Quads of pairs that may pass go to a per-wave LDS queue (entry: grain of
+// the split << 5 | quad of the wave's peaks), and whenever it holds 64 they
+// are settled, one quad per lane, by gs_drlv2.
+// SELECT: cursor = counts; a pair that counts takes a slot of its grain and,
+// when idx is given, writes its peak number there (see k_select_many).
+template <bool SELECT>
+__global__ __launch_bounds__(GS_BLOCK, 4) void k_score_mfma(
+    const double* __restrict__ ubis, int K, int tsplit, int nsplit, const double* __restrict__ gv,
+    int ng, double tolsq, const gs_half8* __restrict__ frag, const float* __restrict__ span,
+    int* __restrict__ counts, const long long* __restrict__ off, int* __restrict__ idx) {
+    constexpr int NW = GS_BLOCK / GS_WAVE;
+    constexpr int NB = GS_SIEVE_SETS;
+    static_assert(8 * NB <= 32, "a queue entry holds 5 bits of quad");
+    static_assert(32 * GS_SIEVE_SPLIT <= 2048, "and 11 bits of grain");
+    __shared__ __align__(16) gs_half8 lpk[NW][NB][GS_WAVE];
+    __shared__ int lcnt[32 * GS_SIEVE_SPLIT];
+    __shared__ unsigned short lq[NW][GS_WAVE + 256];
+    const int tile = gs_xcd_remap(blockIdx.x, gridDim.x);
+    const int chunk = tile / nsplit;
+    const int split = tile - chunk * nsplit;
+    const int t0 = split * tsplit;
+    const int t1 = min((K + 31) / 32, t0 + tsplit);
+    const int g0 = 32 * t0;
+    const int lane = threadIdx.x & (GS_WAVE - 1);
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / GS_WAVE);
+    const int half = lane >> 5;
+    for (int i = threadIdx.x; i < 32 * (t1 - t0); i += GS_BLOCK) lcnt[i] = 0;
+    // this wave's peaks: k0 .. k0 + 32 NB - 1, those past ng repeat the last
+    const long long k0 = (long long)chunk * (NW * NB * 32) + wave * (NB * 32);
+    float gmax = 0.0f;
+    for (int s = 0; s < NB; s++) {
+        long long k = k0 + 32 * s + (lane & 31);
+        k = k < ng ? k : (long long)ng - 1;
+        double x = gv[3 * k], y = gv[3 * k + 1], z = gv[3 * k + 2];
+        if (!(gs_finite(x) && gs_finite(y) && gs_finite(z))) {
+            x = 0.3137;  // a NaN drlv2 in any case: never counted
+            y = 0.2711;
+            z = 0.1873;
+        }
+        gmax = fmaxf(gmax, (float)fmax(fabs(x), fmax(fabs(y), fabs(z))));
+        lpk[wave][s][lane] = gs_peak_frag(x, y, z, nullptr, half);
+    }
+    for (int o = 1; o < 32; o <<= 1) gmax = fmaxf(gmax, __shfl_xor(gmax, o, GS_WAVE));
+    gmax = __builtin_bit_cast(
+        float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, gmax * (1.0f + 0x1p-20f))));
+    const double tol = sqrt(tolsq) * (1.0 + 1e-15) + 1e-12;
+    int r16, thr, r16w, thrw;
+    gs_sieve_units(tol + GS_SIEVE_ERR, r16, thr);
+    gs_sieve_units(tol + GS_SIEVE_ERR_WIDE, r16w, thrw);
+    unsigned short* q = lq[wave];
+    int qn = 0;
+    const auto hit = [&](int gl, long long k) {
+        if constexpr (SELECT) {
+            const int g = g0 + gl;
+            const int slot = atomicAdd(&counts[g], 1);
+            if (idx && slot < off[g + 1] - off[g]) idx[off[g] + slot] = (int)k;
+        } else {
+            atomicAdd(&lcnt[gl], 1);
+        }
+    };
+    const auto settle = [&](unsigned e) {
+        const int gl = e >> 5;
+        if (g0 + gl >= K) return;  // the repeated last grain
+        const gs_ubi u = gs_load_ubi(ubis + 9 * (size_t)(g0 + gl));
+        const long long k = k0 + 4 * (e & 31);
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const long long ki = min(k + i, (long long)ng - 1);  // the repeated last peak
+            if (gs_drlv2(u, gv[3 * ki], gv[3 * ki + 1], gv[3 * ki + 2]) < tolsq && k + i < ng)
+                hit(gl, k + i);
+        }
+    };
+    const auto drain = [&] {
+        while (qn >= GS_WAVE) {
+            qn -= GS_WAVE;
+            __builtin_amdgcn_wave_barrier();
+            settle(q[qn + lane]);
+            __builtin_amdgcn_wave_barrier();
+        }
+    };
+    __syncthreads();
+    const gs_half8* f = frag + 3 * (size_t)t0 * GS_WAVE + lane;
+    gs_half8 n0 = f[0], n1 = f[GS_WAVE], n2 = f[2 * GS_WAVE];
+    const gs_float16 c = gs_splat16(12582912.0f + r16);  // 1.5 2^23
+    for (int t = t0; t < t1; t++) {
+        const gs_half8 b0 = n0, b1 = n1, b2 = n2;
+        const float sp = span[t] * gmax;
+        const bool fits = span[t] < GS_SIEVE_UMAX && gmax < GS_SIEVE_GMAX;
+        if (t + 1 < t1) {  // the next tile's fragments, in flight during this one
+            f += 3 * GS_WAVE;
+            n0 = f[0];
+            n1 = f[GS_WAVE];
+            n2 = f[2 * GS_WAVE];
+        }
+        // entry of quad j, set s: lane part + 8 s + 2 j
+        const unsigned lp = ((32 * (t - t0) + (lane & 31)) << 5) | half;
+        if (fits && sp <= GS_SIEVE_SPAN) {
+#pragma unroll 1
+            for (int s = 0; s < NB; s++) {
+                gs_sieve_tile<false>(lpk[wave][s][lane], b0, b1, b2, c, thr, lp + 8 * s, q, qn);
+                drain();
+            }
+        } else if (fits && sp <= GS_SIEVE_SPAN_WIDE) {
+            const gs_float16 cw = gs_splat16(201326592.0f + r16w);  // 1.5 2^27
+#pragma unroll 1
+            for (int s = 0; s < NB; s++) {
+                gs_sieve_tile<true>(lpk[wave][s][lane], b0, b1, b2, cw, thrw, lp + 8 * s, q, qn);
+                drain();
+            }
+        } else {
+            for (int g = 32 * t; g < min(K, 32 * t + 32); g++) {
+                const gs_ubi u = gs_load_ubi(ubis + 9 * (size_t)g);
+                for (int s = 0; s < NB * 32; s += GS_WAVE) {
+                    const long long k = k0 + s + lane;
+                    if (k < ng && gs_drlv2(u, gv[3 * k], gv[3 * k + 1], gv[3 * k + 2]) < tolsq)
+                        hit(g - g0, k);
+                }
+            }
+        }
+    }
+    __builtin_amdgcn_wave_barrier();
+    if (lane < qn) settle(q[lane]);
+    if constexpr (!SELECT) {
+        __syncthreads();
+        for (int i = threadIdx.x; i < 32 * (t1 - t0); i += GS_BLOCK) {
+            const int c = lcnt[i];
+            if (c) atomicAdd(&counts[g0 + i], c);
+        }
+    }
+}

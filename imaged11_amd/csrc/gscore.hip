@@ -26,6 +26,7 @@
 #include <sched.h>
 
 #include "gs_kernels.h"
+#include "gs_sieve.h"
 #include "gs_adjoint.h"
 #include "gs_assign_gv.h"
 #include "gs_index.h"
@@ -282,6 +283,53 @@ int pair_tiles(DeviceCtx* ctx, int K, int ng, int P, int* gsplit_out, int* nspli
     *gsplit_out = gsplit;
     *nsplit_out = (int)nsplit;
     *nb_out = (unsigned)nb;
+    return GS_OK;
+}
+
+// Blocks of the matrix-core sieve: chunks of 4 x 32 GS_SIEVE_SETS peaks times
+// splits of at most GS_SIEVE_SPLIT grain tiles.  About 16 blocks per CU (4
+// rounds of resident blocks): 4, 8 and 16 measured the same at 1000 x 10^6
+// (146 us), 16 the best at 3000 x 186531 (86 us against 89).
+int sieve_grid(DeviceCtx* ctx, int K, int ng, int* tsplit_out, int* nsplit_out,
+               unsigned* nb_out) {
+    const long long per = 32LL * GS_SIEVE_SETS * (GS_BLOCK / GS_WAVE);
+    const long long nchunks = (ng + per - 1) / per;
+    const long long tiles = gs_sieve_tiles(K);
+    long long nsplit = std::max<long long>(1, (16LL * ctx->cus + nchunks - 1) / nchunks);
+    nsplit = std::min(nsplit, tiles);
+    nsplit = std::max<long long>(nsplit, (tiles + GS_SIEVE_SPLIT - 1) / GS_SIEVE_SPLIT);
+    const long long tsplit = (tiles + nsplit - 1) / nsplit;
+    nsplit = (tiles + tsplit - 1) / tsplit;
+    const long long nb = nchunks * nsplit;
+    if (nb > 0x7fffffffLL) return set_err(GS_ERR_ARG, "grid too large");
+    *tsplit_out = (int)tsplit;
+    *nsplit_out = (int)nsplit;
+    *nb_out = (unsigned)nb;
+    return GS_OK;
+}
+
+// score (idx, off NULL) or list extraction (SELECT) by the matrix-core
+// sieve: the pack launch, which also clears counts, and the pairs.
+template <bool SELECT>
+int launch_sieve(const double* ubis, int K, const double* gv, int ng, double tolsq, int* counts,
+                 const long long* off, int* idx, void* ws, hipStream_t st) {
+    DeviceCtx* ctx;
+    GS_CHECK(get_ctx(&ctx));
+    if (K < 0 || ng < 0) return set_err(GS_ERR_ARG, "negative size K=%d ng=%d", K, ng);
+    if (K == 0 || ng == 0) return fill_i32(counts, 0, K, st);
+    if (!ws || (reinterpret_cast<uintptr_t>(ws) & 15))
+        return set_err(GS_ERR_ARG, "the sieve needs a 16-byte aligned workspace");
+    int tsplit, nsplit;
+    unsigned nb;
+    GS_CHECK(sieve_grid(ctx, K, ng, &tsplit, &nsplit, &nb));
+    const int tiles = (int)gs_sieve_tiles(K);
+    gs_half8* frag = static_cast<gs_half8*>(ws);
+    float* span = reinterpret_cast<float*>(frag + 3 * (size_t)tiles * GS_WAVE);
+    hipLaunchKernelGGL(k_sieve_pack, dim3(tiles), dim3(128), 0, st, ubis, K, frag, span, counts);
+    GS_LAUNCHED();
+    hipLaunchKernelGGL(k_score_mfma<SELECT>, dim3(nb), dim3(GS_BLOCK), 0, st, ubis, K, tsplit,
+                       nsplit, gv, ng, tolsq, frag, span, counts, off, idx);
+    GS_LAUNCHED();
     return GS_OK;
 }
 
@@ -1012,6 +1060,13 @@ int gs_score_many(const double* ubis, int K, const double* gv, int ng, double to
     if (mode != GS_SCORE_CERTIFIED && mode != GS_SCORE_EXACT && mode != GS_SCORE_SIEVE)
         return set_err(GS_ERR_ARG, "gs_score_many: unknown mode %d", mode);
     return launch_score_many(ubis, K, gv, ng, tol, counts, peaks_per_lane, mode, S(stream));
+}
+
+long long gs_sieve_workspace_bytes(int K) { return gs_sieve_ws_bytes(K > 0 ? K : 0); }
+
+int gs_score_many_ws(const double* ubis, int K, const double* gv, int ng, double tol, int* counts,
+                     void* ws, gs_stream_t stream) {
+    return launch_sieve<false>(ubis, K, gv, ng, tol * tol, counts, nullptr, nullptr, ws, S(stream));
 }
 
 int gs_assign_many(const double* ubis, const int* grain_labels, int K, const double* gv, int ng,

@@ -1,0 +1,54 @@
+"""The error bound of the matrix-core sieve, in numpy: h from f16 pieces,
+products exact, f32 accumulation that rounds or truncates at every step."""
+import numpy as np
+import pytest
+
+
+def split16(v):
+    hi = np.float16(np.float32(v))
+    return hi, np.float16(np.float32(v - hi.astype(np.float64)))
+
+
+def accumulate(prods, start, mode, rng):
+    """Sum of the k slots in a random order, every addition rounded to f32
+    to nearest or towards zero."""
+    acc = np.full(prods.shape[0], np.float32(start))
+    for k in rng.permutation(prods.shape[1]):
+        s = acc.astype(np.float64) + prods[:, k]
+        f = s.astype(np.float32)
+        if mode == "truncate":
+            over = np.abs(f.astype(np.float64)) > np.abs(s)
+            f = np.where(over, np.nextafter(f, np.float32(0)), f)
+        acc = f
+    return acc
+
+
+@pytest.mark.parametrize("mode", ["nearest", "truncate"])
+@pytest.mark.parametrize("span,start,err", [(60.0, 1.5 * 2.0 ** 23, 2.0 ** -11),
+                                            (1000.0, 1.5 * 2.0 ** 27, 2.0 ** -7)])
+def test_sieve_error_bound(mode, span, start, err):
+    rng = np.random.default_rng(1)
+    worst = 0.0
+    for scale in (1e-3, 0.3, 4.0, 60.0, 800.0):
+        n = 20000
+        u = rng.uniform(-1, 1, (n, 3)) * scale
+        gmax = min(29.9, span / np.abs(u).sum(1).max())
+        g = rng.uniform(-1, 1, (n, 3)) * gmax
+        g[::7] = np.sign(u[::7]) * gmax  # the largest sums
+        uh, ul = split16(u * 64.0)
+        gh, gl = split16(g * 1024.0)
+        f = lambda a: a.astype(np.float64)
+        prods = np.concatenate([f(gh) * f(uh), f(gl) * f(uh), f(gh) * f(ul)], 1)
+        acc = accumulate(prods, start, mode, rng)
+        assert np.all((acc >= start * 2 / 3) & (acc < start * 4 / 3))  # one binade
+        h = (acc.astype(np.float64) - start) / 65536.0
+        exact = (u.astype(np.longdouble) * g.astype(np.longdouble)).sum(1)
+        worst = max(worst, float(np.abs(h - exact).max()))
+    assert worst < err
+    assert worst > err / 200  # the test reaches the range the bound is for
+
+
+def test_workspace_size_is_the_library_s():
+    from imaged11_amd import _lib
+    for K in (0, 1, 31, 32, 33, 1000, 20000):
+        assert _lib.sieve_ws(K, "cpu").numel() == _lib.load().gs_sieve_workspace_bytes(K)
