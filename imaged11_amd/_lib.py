@@ -51,6 +51,9 @@ SIGNATURES = {
     "gs_sieve_workspace_bytes": (ctypes.c_longlong, [_i]),
     "gs_score_many_ws": (_i, [_vp, _i, _vp, _i, _d, _vp, _vp, _vp]),
     "gs_assign_many": (_i, [_vp, _vp, _i, _vp, _i, _d, _vp, _vp, _vp, _i, _vp]),
+    "gs_assign_many_ws": (_i, [_vp, _i, _vp, _i, _d, _vp, _vp, _vp, _vp, _vp]),
+    "gs_gv_assign_many_ws": (_i, [_vp, _vp, _vp, _i, _d, _d, _d, _dp, _vp, _vp, _i, _d, _vp, _vp,
+                                  _vp, _vp, _vp]),
     "gs_score_and_refine_dev": (_i, [_vp, _vp, _i, _d, _vp, _vp, _vp]),
     "gs_refine_assigned_dev": (_i, [_vp, _vp, _i, _vp, _i, _vp, _vp, _vp]),
     "gs_score_and_refine_dev_noalloc": (_i, [_vp, _vp, _i, _d, _vp, _vp, _vp]),
@@ -237,7 +240,7 @@ def hptr(a):
 def sieve_ws(K, device):
     """Device workspace of the matrix-core sieve for K grains
     (gs_sieve_workspace_bytes(K) bytes)."""
-    return torch.empty((K + 31) // 32 * 3088, dtype=torch.uint8, device=device)
+    return torch.empty((K + 31) // 32 * 3088 + 16, dtype=torch.uint8, device=device)
 
 
 def darr(values):

@@ -47,6 +47,15 @@ def mfma_pays(K, N):
     return K >= 24 and K * N >= 12000000
 
 
+def assign_mfma_pays(K, N, tol):
+    """Whether the assignment behind the matrix-core sieve is the faster one
+    for K grains x N peaks.  A peak's fragments cost as much as ~10 grains of
+    the FP64 loop (10 x 8e6 with positions: 280 us against 172, 16 x 1e6: 39
+    against 41, 777 x 10^5: 90 against 337), and beyond tol 0.12 too many pairs
+    pass (500 x 200003: 240 us against 351 at 0.1, 449 against 401 at 0.15)."""
+    return K >= 16 and abs(float(tol)) <= SIEVE_TOL_MAX
+
+
 def score_sieve(ubis, gv, tol, out=None):
     """score_many by the sieve on the matrix cores (gs_score_many_ws), at any
     size and tolerance."""
@@ -113,11 +122,18 @@ def assign_many(ubis, gv, tol, drlv2, labels, grain_labels=None, out=None, exact
     K = ubis.shape[0]
     _need(drlv2, torch.float64, "drlv2", (N,))
     _need(labels, torch.int32, "labels", (N,))
+    if out is None:
+        out = torch.empty(K, dtype=torch.int32, device=gv.device)
+    if grain_labels is None and not exact and assign_mfma_pays(K, N, tol):
+        _need(out, torch.int32, "out", (K,))
+        ws = _lib.sieve_ws(K, gv.device)
+        _lib.check(lib.gs_assign_many_ws(dptr(ubis), K, dptr(gv), N, float(tol), dptr(drlv2),
+                                         dptr(labels), dptr(out), dptr(ws), stream_ptr()),
+                   "assign_many")
+        return out
     if grain_labels is None:
         grain_labels = torch.arange(K, dtype=torch.int32, device=gv.device)
     _need(grain_labels, torch.int32, "grain_labels", (K,))
-    if out is None:
-        out = torch.empty(K, dtype=torch.int32, device=gv.device)
     mode = _lib.SCORE_EXACT if exact else _lib.SCORE_CERTIFIED
     _lib.check(lib.gs_assign_many(dptr(ubis), dptr(grain_labels), K, dptr(gv), N, float(tol),
                                   dptr(drlv2), dptr(labels), dptr(out), mode, stream_ptr()),
@@ -327,11 +343,19 @@ def gv_assign_many(xl, so, co, wvln, ubis, trans, tol, drlv2, labels, grain_labe
     _need(trans, torch.float64, "trans", (K, 3))
     _need(drlv2, torch.float64, "drlv2", (N,))
     _need(labels, torch.int32, "labels", (N,))
+    if out is None:
+        out = torch.empty(K, dtype=torch.int32, device=xl.device)
+    if grain_labels is None and assign_mfma_pays(K, N, tol):
+        _need(out, torch.int32, "out", (K,))
+        ws = _lib.sieve_ws(K, xl.device)
+        _lib.check(lib.gs_gv_assign_many_ws(dptr(xl), dptr(so), dptr(co), N, float(wvln),
+                                            float(wedge), float(chi), _mat_arg(mat), dptr(ubis),
+                                            dptr(trans), K, float(tol), dptr(drlv2), dptr(labels),
+                                            dptr(out), dptr(ws), stream_ptr()), "gv_assign_many")
+        return out
     if grain_labels is None:
         grain_labels = torch.arange(K, dtype=torch.int32, device=xl.device)
     _need(grain_labels, torch.int32, "grain_labels", (K,))
-    if out is None:
-        out = torch.empty(K, dtype=torch.int32, device=xl.device)
     _lib.check(lib.gs_gv_assign_many(dptr(xl), dptr(so), dptr(co), N, float(wvln), float(wedge),
                                      float(chi), _mat_arg(mat), dptr(ubis), dptr(trans),
                                      dptr(grain_labels), K, float(tol), dptr(drlv2), dptr(labels),

@@ -137,10 +137,10 @@ __device__ __forceinline__ unsigned short gs_sieve_field(float a, float b, float
 // where it passes the quad is appended to the wave's queue, entry lp + 2 j.
 // The queue's fill qn is wave-uniform; at most 256 entries are added, in
 // order of j, then lane.
-template <bool WIDE>
+template <bool WIDE, class Entry>
 __device__ __forceinline__ void gs_sieve_tile(gs_half8 pk, gs_half8 b0, gs_half8 b1, gs_half8 b2,
                                               gs_float16 c, unsigned short thr, unsigned lp,
-                                              unsigned short* q, int& qn) {
+                                              Entry* q, int& qn) {
     const gs_float16 h0 = __builtin_amdgcn_mfma_f32_32x32x16_f16(pk, b0, c, 0, 0, 0);
     const gs_float16 h1 = __builtin_amdgcn_mfma_f32_32x32x16_f16(pk, b1, c, 0, 0, 0);
     const gs_float16 h2 = __builtin_amdgcn_mfma_f32_32x32x16_f16(pk, b2, c, 0, 0, 0);
@@ -158,7 +158,7 @@ __device__ __forceinline__ void gs_sieve_tile(gs_half8 pk, gs_half8 b0, gs_half8
             if (in) {
                 const unsigned pos = __builtin_amdgcn_mbcnt_hi(
                     (unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u));
-                (q + qn)[pos] = (unsigned short)(lp + 2 * j);
+                (q + qn)[pos] = (Entry)(lp + 2 * j);
             }
             qn += __popcll(m);
         }
@@ -176,7 +176,7 @@ __device__ __forceinline__ gs_float16 gs_splat16(float v) {
 // slots 8 (l >> 5) .. + 7, then one float per tile, the largest row sum of
 // |u|.  Also clears counts (so that no separate fill is launched).
 inline long long gs_sieve_tiles(long long K) { return (K + 31) / 32; }
-inline long long gs_sieve_ws_bytes(long long K) { return gs_sieve_tiles(K) * (3 * 64 * 16 + 16); }
+inline long long gs_sieve_ws_bytes(long long K) { return gs_sieve_tiles(K) * (3 * 64 * 16 + 16) + 16; }
 
 __global__ __launch_bounds__(128) void k_sieve_pack(const double* __restrict__ ubis, int K,
                                                     gs_half8* __restrict__ frag,

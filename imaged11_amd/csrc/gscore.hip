@@ -29,6 +29,7 @@
 #include "gs_sieve.h"
 #include "gs_adjoint.h"
 #include "gs_assign_gv.h"
+#include "gs_assign_mfma.h"
 #include "gs_index.h"
 #include "gs_geometry.h"
 #include "gs_grains.h"
@@ -402,6 +403,52 @@ int launch_assign_many(const double* ubis, const int* glabels, int K, const doub
                            glabels, K, gv, ng, tolsq, drlv2, labels, counts);
     GS_LAUNCHED();
     return GS_OK;
+}
+
+// score_and_assign for grains 0..K-1 with label g for grain g, by the
+// matrix-core sieve: the pack launch, which also clears counts, and the
+// pairs.  32, 64 or 128 peaks per wave: the largest that still gives every
+// SIMD two waves.
+template <bool GEOM, int NB>
+int launch_assign_nb(const double* gvx, const double* so, const double* co, int ng,
+                     const gs_goniometer& gp, const double* ubis, const double* trans, int K,
+                     double tolsq, const gs_half8* frag, const gs_tile_info* info,
+                     const int* yexp, double* drlv2, int* labels, int* counts, hipStream_t st) {
+    const int nb = blocks_for(ng, 32 * NB * (GS_BLOCK / GS_WAVE));
+    hipLaunchKernelGGL((k_assign_mfma<GEOM, NB>), dim3(nb), dim3(GS_BLOCK), 0, st, gvx, so, co, ng,
+                       gp, ubis, trans, K, tolsq, frag, info, yexp, drlv2, labels, counts);
+    GS_LAUNCHED();
+    return GS_OK;
+}
+
+template <bool GEOM>
+int launch_assign_sieve(const double* gvx, const double* so, const double* co, int ng,
+                        const gs_goniometer& gp, const double* ubis, const double* trans, int K,
+                        double tol, double* drlv2, int* labels, int* counts, void* ws,
+                        hipStream_t st) {
+    DeviceCtx* ctx;
+    GS_CHECK(get_ctx(&ctx));
+    if (K < 0 || ng < 0) return set_err(GS_ERR_ARG, "negative size K=%d ng=%d", K, ng);
+    if (K > (1 << 24)) return set_err(GS_ERR_ARG, "the assignment sieve takes at most 2^24 grains");
+    if (K == 0 || ng == 0) return fill_i32(counts, 0, K, st);
+    if (!ws || (reinterpret_cast<uintptr_t>(ws) & 15))
+        return set_err(GS_ERR_ARG, "the sieve needs a 16-byte aligned workspace");
+    const int tiles = (int)gs_sieve_tiles(K);
+    gs_half8* frag = static_cast<gs_half8*>(ws);
+    gs_tile_info* info = reinterpret_cast<gs_tile_info*>(frag + 3 * (size_t)tiles * GS_WAVE);
+    int* yexp = reinterpret_cast<int*>(info + tiles);
+    hipLaunchKernelGGL(k_assign_pack<GEOM>, dim3(tiles), dim3(128), 0, st, ubis, trans, K, frag,
+                       info, yexp, counts);
+    GS_LAUNCHED();
+    const long long waves = 8LL * ctx->cus;
+    if (ng >= 128 * waves)
+        return launch_assign_nb<GEOM, 4>(gvx, so, co, ng, gp, ubis, trans, K, tol * tol, frag, info,
+                                         yexp, drlv2, labels, counts, st);
+    if (ng >= 64 * waves)
+        return launch_assign_nb<GEOM, 2>(gvx, so, co, ng, gp, ubis, trans, K, tol * tol, frag, info,
+                                         yexp, drlv2, labels, counts, st);
+    return launch_assign_nb<GEOM, 1>(gvx, so, co, ng, gp, ubis, trans, K, tol * tol, frag, info,
+                                     yexp, drlv2, labels, counts, st);
 }
 
 // Blocks of the one-grain refinement: one per 4·GS_BLOCK peaks, at most
@@ -1078,6 +1125,12 @@ int gs_assign_many(const double* ubis, const int* grain_labels, int K, const dou
                               S(stream));
 }
 
+int gs_assign_many_ws(const double* ubis, int K, const double* gv, int ng, double tol,
+                      double* drlv2, int* labels, int* counts, void* ws, gs_stream_t stream) {
+    return launch_assign_sieve<false>(gv, nullptr, nullptr, ng, gs_goniometer(), ubis, nullptr, K,
+                                      tol, drlv2, labels, counts, ws, S(stream));
+}
+
 int gs_score_and_refine_dev(double* ubi, const double* gv, int ng, double tol, int* n_out,
                             double* mean_out, gs_stream_t stream) {
     return launch_refine_one(0, ubi, gv, ng, tol, nullptr, 0, n_out, mean_out, S(stream));
@@ -1576,6 +1629,15 @@ int gs_gv_assign_many(const double* xlylzl, const double* so, const double* co, 
                        co, ng, gp, ubis, trans, grain_labels, K, tol * tol, drlv2, labels, counts);
     GS_LAUNCHED();
     return GS_OK;
+}
+
+int gs_gv_assign_many_ws(const double* xlylzl, const double* so, const double* co, int ng,
+                         double wvln, double wedge, double chi, const double* mat,
+                         const double* ubis, const double* trans, int K, double tol,
+                         double* drlv2, int* labels, int* counts, void* ws, gs_stream_t stream) {
+    return launch_assign_sieve<true>(xlylzl, so, co, ng,
+                                     make_gonio(1.0, wvln, wedge, chi, nullptr, mat), ubis, trans,
+                                     K, tol, drlv2, labels, counts, ws, S(stream));
 }
 
 int gs_gv_lists(const double* xlylzl, const double* so, const double* co, int ng, double wvln,

@@ -149,6 +149,12 @@ int gs_assign_many(const double *ubis, const int *grain_labels, int K, const dou
                    int ng, double tol, double *drlv2, int *labels, int *counts, int mode,
                    gs_stream_t stream);
 
+/* The same with label g for grain g (grain_labels = 0..K-1) and the sieve on
+ * the matrix cores in front (same results at any tol; its fastest form for
+ * |tol| <= 0.1).  ws as for gs_score_many_ws; K <= 2^24. */
+int gs_assign_many_ws(const double *ubis, int K, const double *gv, int ng, double tol,
+                      double *drlv2, int *labels, int *counts, void *ws, gs_stream_t stream);
+
 /* one-grain score_and_refine / refine_assigned on device memory; ubi (9
  * doubles) is updated in place, n_out/mean_out are device scalars. */
 int gs_score_and_refine_dev(double *ubi, const double *gv, int ng, double tol, int *n_out,
@@ -373,6 +379,12 @@ int gs_gv_assign_many(const double *xlylzl, const double *so, const double *co, 
                       double wvln, double wedge, double chi, const double *mat,
                       const double *ubis, const double *trans, const int *grain_labels, int K,
                       double tol, double *drlv2, int *labels, int *counts, gs_stream_t stream);
+/* The same with label g for grain g, as gs_assign_many_ws. */
+int gs_gv_assign_many_ws(const double *xlylzl, const double *so, const double *co, int ng,
+                         double wvln, double wedge, double chi, const double *mat,
+                         const double *ubis, const double *trans, int K, double tol,
+                         double *drlv2, int *labels, int *counts, void *ws, gs_stream_t stream);
+
 
 /* out[q] = compute_gv of peak idx[q] for the translation of grain owner[q]
  * (n_idx rows of 3); rows with an out-of-range index are NaN. */

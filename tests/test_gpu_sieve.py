@@ -114,3 +114,105 @@ def test_graph_replays_equal_the_eager_counts(dev):
         torch.cuda.synchronize()
         got = out.clone()
         assert torch.equal(got, batched.score_many(u, g, 0.05, exact=True))
+
+
+# ---- assignment ------------------------------------------------------------
+
+
+def scan_inputs(K, N, seed, dist=150000.0, t=200.0, cell=(3.0, 9.0), wvln=0.2):
+    rng = np.random.default_rng(seed)
+    ubi = np.linalg.inv(simulate.random_rotations(K, rng) /
+                        rng.uniform(*cell, size=(K, 3))[:, None, :])
+    trans = rng.uniform(-t, t, size=(K, 3)) if t else np.zeros((K, 3))
+    ang = rng.uniform(0, 0.35, N)
+    eta = rng.uniform(0, 2 * np.pi, N)
+    xl = dist / np.cos(ang)[:, None] * np.stack([np.cos(ang), np.sin(ang) * np.cos(eta),
+                                                 np.sin(ang) * np.sin(eta)], 1)
+    om = rng.uniform(-np.pi, np.pi, N)
+    return ubi, trans, xl, np.sin(om), np.cos(om), wvln, rng
+
+
+def check_scan(dev, orc, ubi, trans, xl, so, co, wvln, tol, d0, l0, mat=None):
+    """gv_assign_many with default labels (the sieve) against the oracle's loop."""
+    K = len(ubi)
+    mat = np.eye(3) if mat is None else mat
+    d, lab = d0.copy(), l0.copy()
+    want = orc.gv_assign_many(xl, so, co, mat, wvln, ubi, trans, np.arange(K), tol, d, lab)
+    dd, ll = T(d0, dev), T(l0, dev, torch.int32)
+    assert batched.assign_mfma_pays(K, len(xl), tol)
+    got = batched.gv_assign_many(T(xl, dev), T(so, dev), T(co, dev), wvln, T(ubi, dev),
+                                 T(trans, dev), tol, dd, ll, mat=mat)
+    assert np.array_equal(got.cpu().numpy(), want)
+    assert np.array_equal(ll.cpu().numpy(), lab)
+    assert np.array_equal(dd.cpu().numpy().view(np.int64), d.view(np.int64))
+    return want
+
+
+@pytest.mark.parametrize("K,N", [(16, 1), (16, 31), (31, 32), (32, 33), (33, 127), (64, 129),
+                                 (65, 511), (2049, 600), (20, 140000), (17, 270001)])
+def test_scan_at_tile_edges(dev, orc, K, N):
+    ubi, trans, xl, so, co, w, rng = scan_inputs(K, N, K + N)
+    check_scan(dev, orc, ubi, trans, xl, so, co, w, 0.1, np.ones(N), np.full(N, -1, np.int32))
+
+
+# positions from none to as large as the detector distance (micron and other
+# units), so that tiles are sieved, sieved with a wide radius, or not at all
+@pytest.mark.parametrize("dist,t", [(150000.0, 0.0), (150000.0, 1000.0), (150000.0, 6000.0),
+                                    (150000.0, 20000.0), (8000.0, 300.0), (5000.0, 2600.0),
+                                    (150.0, 0.2), (0.15, 2e-4), (150000.0, 200000.0)])
+@pytest.mark.parametrize("cell", [(3.0, 9.0), (20.0, 45.0), (300.0, 1200.0)])
+def test_scan_over_positions_and_cells(dev, orc, dist, t, cell):
+    ubi, trans, xl, so, co, w, rng = scan_inputs(100, 3000, 4, dist=dist, t=t, cell=cell)
+    mat = orc.wedge_chi_matrix(1.5, -2.0).reshape(3, 3)
+    want = check_scan(dev, orc, ubi, trans, xl, so, co, w, 0.1, np.ones(3000),
+                      np.full(3000, -1, np.int32), mat)
+    assert want.sum() > 300
+
+
+def test_scan_from_other_states(dev, orc):
+    """Labels of the grains and others, current drlv2 anywhere in reach,
+    repeated grains, peaks and grains with special values, a peak at the
+    origin."""
+    K, N = 150, 5000
+    ubi, trans, xl, so, co, w, rng = scan_inputs(K, N, 8)
+    ubi[70:90], trans[70:90] = ubi[50:70], trans[50:70]  # equal drlv2: the first keeps the peak
+    for i, v in enumerate([np.nan, np.inf, 1e300, 0.0]):
+        xl[11 * i] = v
+        xl[11 * i + 3, i % 3] = v
+        ubi[5 * i, 1, 2] = v
+        trans[5 * i + 40, i % 3] = v
+        so[11 * i + 5] = v
+    l0 = rng.integers(-3, K + 5, N).astype(np.int32)
+    d0 = rng.uniform(0.0, 0.02, N)
+    d0[::13] = np.nan
+    d0[1::13] = np.inf
+    check_scan(dev, orc, ubi, trans, xl, so, co, w, 0.1, d0, l0)
+
+
+@pytest.mark.parametrize("tol", [0.001, 0.05, 0.1])
+@pytest.mark.parametrize("K,N", [(16, 1), (33, 129), (300, 20001), (2100, 300)])
+def test_assignment_of_gvectors(dev, orc, K, N, tol):
+    ubi, gv = make(K, N, K)
+    rng = np.random.default_rng(K)
+    for d0, l0 in ((np.full(N, 2.0), np.full(N, -1, np.int32)),
+                   (rng.uniform(0, 0.02, N), rng.integers(-2, K + 2, N).astype(np.int32))):
+        d, lab = d0.copy(), l0.copy()
+        want = orc.assign_many(ubi, np.arange(K), gv, tol, d, lab)
+        dd, ll = T(d0, dev), T(l0, dev, torch.int32)
+        got = batched.assign_many(T(ubi, dev), T(gv, dev), tol, dd, ll)
+        assert np.array_equal(got.cpu().numpy(), want)
+        assert np.array_equal(ll.cpu().numpy(), lab)
+        assert np.array_equal(dd.cpu().numpy().view(np.int64), d.view(np.int64))
+
+
+@pytest.mark.parametrize("cell,gmax", [((20.0, 60.0), 1.6), ((300.0, 900.0), 1.6),
+                                       ((0.05, 0.2), 40.0)])
+def test_assignment_over_the_ranges_of_the_accumulator(dev, orc, cell, gmax):
+    ubi, gv = make(90, 2000, 6, cell=cell, gmax=gmax)
+    d, lab = np.ones(2000), np.full(2000, -1, np.int32)
+    want = orc.assign_many(ubi, np.arange(90), gv, 0.1, d, lab)
+    dd, ll = T(np.ones(2000), dev), T(np.full(2000, -1), dev, torch.int32)
+    got = batched.assign_many(T(ubi, dev), T(gv, dev), 0.1, dd, ll)
+    assert want.sum() > 0 and np.array_equal(got.cpu().numpy(), want)
+    assert np.array_equal(ll.cpu().numpy(), lab)
+    assert np.array_equal(dd.cpu().numpy().view(np.int64), d.view(np.int64))

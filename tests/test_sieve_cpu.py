@@ -52,3 +52,34 @@ def test_workspace_size_is_the_library_s():
     from imaged11_amd import _lib
     for K in (0, 1, 31, 32, 33, 1000, 20000):
         assert _lib.sieve_ws(K, "cpu").numel() == _lib.load().gs_sieve_workspace_bytes(K)
+
+
+@pytest.mark.parametrize("ratio", [1e-4, 2e-3, 0.03, 0.1, 0.2])
+def test_position_expansion_error_bound(ratio):
+    """u.G for a grain at t against the sieve's terms: G0 and the products p q
+    with p and q rounded to f16, over t/|a| up to the largest sieved."""
+    rng = np.random.default_rng(2)
+    n, ds, amin = 20000, 5.0, 150000.0
+    a = rng.normal(size=(n, 3))
+    a *= (amin * rng.uniform(1.0, 1.3, n) / np.linalg.norm(a, axis=1))[:, None]
+    t = rng.normal(size=(n, 3))
+    t *= (ratio * amin * rng.uniform(0.0, 1.0, n) / np.linalg.norm(t, axis=1))[:, None]
+    t[::5] = np.cross(a[::5], [0.3, -0.5, 0.8])  # across the beam: the largest remainder
+    t[::5] *= ratio * amin / np.linalg.norm(t[::5], axis=1)[:, None]
+    u = rng.uniform(-9, 9, (n, 3))
+    e = a - t
+    exact = (u * (ds * e / np.linalg.norm(e, axis=1)[:, None])).sum(1)
+    r = np.linalg.norm(a, axis=1)
+    nn = a / r[:, None]
+    i, j = np.array([0, 1, 2, 0, 0, 1]), np.array([0, 1, 2, 1, 2, 2])
+    y = 4 - int(np.frexp(np.abs(t).max())[1])
+    p = (ds / r)[:, None] * nn[:, i] * nn[:, j]
+    q = u[:, i] * t[:, j] + u[:, j] * t[:, i]
+    q[:, :3] = u * t - (u * t).sum(1)[:, None]
+    p16 = np.float16(np.float32(p * 2.0 ** (16 - y))).astype(float)
+    q16 = np.float16(np.float32(q * 2.0 ** y)).astype(float)
+    assert p16.max() < 8192 and np.isfinite(q16).all()
+    approx = (u * (ds * nn)).sum(1) + (p16 * q16).sum(1) / 65536.0
+    L, A1, T = np.abs(q).sum(1), np.abs(u).sum(1), np.linalg.norm(t, axis=1)
+    bound = 1.01 * 2.0 ** -10 * ds / amin * L + 0.5775 * A1 * ds * (T / (amin - T)) ** 2
+    assert np.all(np.abs(approx - exact) <= bound + 1e-12)
