@@ -49,6 +49,7 @@ SIGNATURES = {
     "compute_xlylzl": (None, [_vp, _vp, _vp, _vp, _vp, _vp, _i]),
     "gs_score_many": (_i, [_vp, _i, _vp, _i, _d, _vp, _i, _i, _vp]),
     "gs_sieve_workspace_bytes": (ctypes.c_longlong, [_i]),
+    "gs_assign_workspace_bytes": (ctypes.c_longlong, [_i]),
     "gs_score_many_ws": (_i, [_vp, _i, _vp, _i, _d, _vp, _vp, _vp]),
     "gs_assign_many": (_i, [_vp, _vp, _i, _vp, _i, _d, _vp, _vp, _vp, _i, _vp]),
     "gs_assign_many_ws": (_i, [_vp, _i, _vp, _i, _d, _vp, _vp, _vp, _vp, _vp]),
@@ -85,6 +86,10 @@ SIGNATURES = {
     "gs_graph_launch": (_i, [_vp, _vp]),
     "gs_gv_assign_many": (_i, [_vp, _vp, _vp, _i, _d, _d, _d, _dp, _vp, _vp, _vp, _i, _d, _vp, _vp,
                                _vp, _vp]),
+    "gs_label_counts": (_i, [_vp, _i, _i, _vp, _vp]),
+    "gs_list_offsets": (_i, [_vp, _i, _vp, _vp, _vp, _vp]),
+    "gs_list_fill": (_i, [_vp, _i, _i, _vp, _vp, ctypes.c_longlong, _vp, _vp, _vp]),
+    "gs_list_order": (_i, [_vp, _i, _vp, _vp]),
     "gs_gv_lists": (_i, [_vp, _vp, _vp, _i, _d, _d, _d, _dp, _vp, _i, _vp, _vp, ctypes.c_longlong,
                          _vp, _vp]),
     "gs_joint_hkl": (_i, [_vp, _vp, _vp, _vp, _i, _vp, _vp, _vp, _i, _vp, _vp, ctypes.c_longlong,
@@ -138,6 +143,10 @@ SCORE_CERTIFIED = 0
 SCORE_EXACT = 1
 SCORE_SIEVE = 2
 SIEVE_TOL_MAX = 0.1  # the sieves pay while few of the pairs pass them
+
+
+LIST_SORT_MAX = 16384  # longest list gs_list_fill sorts
+ORDER_MAX = 8192       # most grains gs_list_order takes
 
 
 def score_mode(tol):
@@ -240,7 +249,13 @@ def hptr(a):
 def sieve_ws(K, device):
     """Device workspace of the matrix-core sieve for K grains
     (gs_sieve_workspace_bytes(K) bytes)."""
-    return torch.empty((K + 31) // 32 * 3088 + 16, dtype=torch.uint8, device=device)
+    return torch.empty(load().gs_sieve_workspace_bytes(K), dtype=torch.uint8, device=device)
+
+
+def assign_ws(K, device):
+    """Device workspace of the assignment behind the sieve
+    (gs_assign_workspace_bytes(K) bytes)."""
+    return torch.empty(load().gs_assign_workspace_bytes(K), dtype=torch.uint8, device=device)
 
 
 def darr(values):

@@ -40,11 +40,11 @@ from ._lib import SIEVE_TOL_MAX, score_mode  # noqa: E402  (the default score ke
 
 def mfma_pays(K, N):
     """Whether the matrix-core sieve is the faster one for K grains x N
-    peaks.  Its tiles hold 32 grains, and its workspace costs the host 1.4 us
-    a call: at 16 x 1e6 both sieves take 30 us, below 1e7 pairs both are
-    bound by the host (13.5 us against 14.9 at 300 x 10^4, 23.2 against 17.2
-    at 1000 x 3 10^4)."""
-    return K >= 24 and K * N >= 12000000
+    peaks.  Its tiles hold 32 grains (4 x 10^6: 20 us against 18 of the row
+    sieve, 16 x 10^6: 20 against 31), and its workspace and launches cost the
+    host 1.5 to 4 us a call, which is all there is to a small problem (300 x
+    30 000: 18 us against 14, 1000 x 30 000: 17 against 23)."""
+    return K >= 8 and K * N >= 16000000
 
 
 def assign_mfma_pays(K, N, tol):
@@ -126,7 +126,7 @@ def assign_many(ubis, gv, tol, drlv2, labels, grain_labels=None, out=None, exact
         out = torch.empty(K, dtype=torch.int32, device=gv.device)
     if grain_labels is None and not exact and assign_mfma_pays(K, N, tol):
         _need(out, torch.int32, "out", (K,))
-        ws = _lib.sieve_ws(K, gv.device)
+        ws = _lib.assign_ws(K, gv.device)
         _lib.check(lib.gs_assign_many_ws(dptr(ubis), K, dptr(gv), N, float(tol), dptr(drlv2),
                                          dptr(labels), dptr(out), dptr(ws), stream_ptr()),
                    "assign_many")
@@ -259,7 +259,13 @@ def sf2gv(sc, fc, omega, pars, t=(0.0, 0.0, 0.0), keep=False, parity=False):
 
 
 def list_order(off):
-    """Grain visiting order for the persistent refine: longest list first."""
+    """Grain visiting order for the persistent refine: longest list first,
+    equal lengths in grain order."""
+    K = off.numel() - 1
+    if off.is_cuda and off.dtype == torch.int64 and off.is_contiguous() and 0 < K <= _lib.ORDER_MAX:
+        order = torch.empty(K, dtype=torch.int32, device=off.device)
+        _lib.check(_ready().gs_list_order(dptr(off), K, dptr(order), stream_ptr()), "list_order")
+        return order
     lengths = off[1:] - off[:-1]
     return torch.argsort(lengths, descending=True, stable=True).to(torch.int32)
 
@@ -347,7 +353,7 @@ def gv_assign_many(xl, so, co, wvln, ubis, trans, tol, drlv2, labels, grain_labe
         out = torch.empty(K, dtype=torch.int32, device=xl.device)
     if grain_labels is None and assign_mfma_pays(K, N, tol):
         _need(out, torch.int32, "out", (K,))
-        ws = _lib.sieve_ws(K, xl.device)
+        ws = _lib.assign_ws(K, xl.device)
         _lib.check(lib.gs_gv_assign_many_ws(dptr(xl), dptr(so), dptr(co), N, float(wvln),
                                             float(wedge), float(chi), _mat_arg(mat), dptr(ubis),
                                             dptr(trans), K, float(tol), dptr(drlv2), dptr(labels),
@@ -363,10 +369,42 @@ def gv_assign_many(xl, so, co, wvln, ubis, trans, tol, drlv2, labels, grain_labe
     return out
 
 
+def _int32_labels(labels):
+    return (labels.is_cuda and labels.dtype == torch.int32 and labels.dim() == 1
+            and labels.is_contiguous() and labels.numel() < 2 ** 31)
+
+
+def label_counts(labels, K):
+    """Number of peaks with each label 0..K-1 (int32 (K,))."""
+    if _int32_labels(labels):
+        counts = torch.empty(K, dtype=torch.int32, device=labels.device)
+        _lib.check(_ready().gs_label_counts(dptr(labels), labels.numel(), K, dptr(counts),
+                                            stream_ptr()), "label_counts")
+        return counts
+    lab = labels.long()
+    return torch.bincount(lab[(lab >= 0) & (lab < K)], minlength=K).to(torch.int32)
+
+
 def lists_from_labels(labels, K):
     """CSR peak lists of grains 0..K-1 from per-peak labels (peaks in
     ascending order inside each list, label -1 and others dropped):
     returns (idx int32, off int64 (K+1,), owner int32)."""
+    if _int32_labels(labels) and labels.numel() and K:
+        lib = _ready()
+        dev, n = labels.device, labels.numel()
+        counts = label_counts(labels, K)
+        off = torch.empty(K + 1, dtype=torch.int64, device=dev)
+        cursor = torch.empty(K, dtype=torch.int32, device=dev)
+        info = torch.empty(2, dtype=torch.int64, device=dev)
+        _lib.check(lib.gs_list_offsets(dptr(counts), K, dptr(off), dptr(cursor), dptr(info),
+                                       stream_ptr()), "list_offsets")
+        total, longest = info.tolist()
+        if longest <= _lib.LIST_SORT_MAX:
+            idx = torch.empty(total, dtype=torch.int32, device=dev)
+            owner = torch.empty(total, dtype=torch.int32, device=dev)
+            _lib.check(lib.gs_list_fill(dptr(labels), n, K, dptr(off), dptr(cursor), longest,
+                                        dptr(idx), dptr(owner), stream_ptr()), "list_fill")
+            return idx, off, owner
     lab = labels.long()
     keep = (lab >= 0) & (lab < K)
     peaks = torch.nonzero(keep, as_tuple=False).flatten()

@@ -38,9 +38,8 @@
 //
 // Measured, labels, drlv2 and counts identical: 20 000 grains x 8 10^6 peaks
 // with positions 24.9 ms against 191 of k_gv_assign_many (FP64 VALU, 92%
-// busy), 777 x 10^5 78 us against 336; g-vectors given, 500 x 200 003 with the
-// caller's fills and counts 241 us against 359, 3000 x 500 003 at tol 0.02
-// 0.33 ms against 2.04.  Per 32 x 32 tile: 51 vector instructions for the
+// busy), 777 x 10^5 45 us against 310; g-vectors given, 500 x 200 003 36 us
+// against 230.  Per 32 x 32 tile: 51 vector instructions for the
 // sieve, 23 for pushes, settling and the tile's constants (the accumulator
 // start is rebuilt for each tile: kept across tiles in registers it made the
 // compiler copy and spill it, 37.7 ms), 421 cycles in all; bound, as the score,
@@ -69,17 +68,18 @@ __device__ __forceinline__ float gs_uniform(float v) {
     return __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, v)));
 }
 
-// Fragments and tile_info of every tile, the exponent y, counts cleared.
+// Fragments and tile_info of every tile, the exponent y, the counters cleared.
 template <bool GEOM>
 __global__ __launch_bounds__(128) void k_assign_pack(const double* __restrict__ ubis,
                                                      const double* __restrict__ trans, int K,
                                                      gs_half8* __restrict__ frag,
                                                      gs_tile_info* __restrict__ info,
                                                      int* __restrict__ yexp,
-                                                     int* __restrict__ counts) {
+                                                     int* __restrict__ priv, int copies) {
     __shared__ float lspan[128], llin[128], lt[128];
     const int tl = blockIdx.x, t = threadIdx.x;
-    if (t < 32 && 32 * tl + t < K) counts[32 * tl + t] = 0;
+    if (32 * tl + (t & 31) < K)
+        for (int c = t / 32; c < copies; c += 4) priv[(size_t)c * K + 32 * tl + (t & 31)] = 0;
     int y = 0;
     if constexpr (GEOM) {  // 2^y from the largest |t| component of all grains
         float m = 0.0f;
@@ -149,7 +149,8 @@ __global__ __launch_bounds__(GS_BLOCK, 3) void k_assign_mfma(
     const double* __restrict__ co_in, int ng, gs_goniometer gp, const double* __restrict__ ubis,
     const double* __restrict__ trans, int K, double tolsq, const gs_half8* __restrict__ frag,
     const gs_tile_info* __restrict__ info, const int* __restrict__ yexp,
-    double* __restrict__ drlv2, int* __restrict__ labels, int* __restrict__ counts) {
+    double* __restrict__ drlv2, int* __restrict__ labels, int* __restrict__ priv, int copies) {
+    int* counts = priv + (size_t)(blockIdx.x % copies) * K;  // this block's copy
     constexpr int NW = GS_BLOCK / GS_WAVE;
     constexpr int NP = 32 * NB;  // peaks per wave
     static_assert(NP <= 128, "a queue entry holds 5 bits of quad, 7 of peak");

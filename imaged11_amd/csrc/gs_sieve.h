@@ -170,21 +170,47 @@ __device__ __forceinline__ gs_float16 gs_splat16(float v) {
 }
 
 // ---------------------------------------------------------------------------
+// Counters.  Atomics on one address from all over the chip go one after the
+// other, so the pairs are counted in private copies of the K counters, copy
+// blockIdx % copies for a block, which a last launch sums: a multiple of 8, so
+// that each copy is the business of one XCD, 8 to 64, up to 32768 counters in
+// all.  The assignment of 500 grains over 200 003 peaks took 112 us with one
+// copy and 36 with 64, the score of 24 x 10^6 31 us and 21, of 100 x 10^6 49
+// and 38; of 500 x 3 10^5 both took 43, and from there the score counts in
+// place (147 us against 152 at 1000 x 10^6, the sum's launch).
+#define GS_SCORE_COPIES_MAX 256
+inline int gs_copies(int K) {
+    const int c = 4096 / (K > 0 ? K : 1);
+    return 8 * (c < 1 ? 1 : c > 8 ? 8 : c);
+}
+
+__global__ __launch_bounds__(GS_BLOCK) void k_sum_copies(const int* __restrict__ priv, int copies,
+                                                         int K, int* __restrict__ counts) {
+    const int g = blockIdx.x * GS_BLOCK + threadIdx.x;
+    if (g >= K) return;
+    int s = 0;
+#pragma unroll 8
+    for (int c = 0; c < copies; c++) s += priv[(size_t)c * K + g];  // a multiple of 8
+    counts[g] = s;
+}
+
+// ---------------------------------------------------------------------------
 // The grains' fragments, packed once per call into the caller's workspace:
 // tile t (grains 32 t .. 32 t + 31; past K the last grain again) has
 // 3 x 64 x 16 bytes, row-major by UBI row, lane l holding column l & 31 and k
 // slots 8 (l >> 5) .. + 7, then one float per tile, the largest row sum of
-// |u|.  Also clears counts (so that no separate fill is launched).
+// |u|.  Also clears the counters (so that no separate fill is launched).
 inline long long gs_sieve_tiles(long long K) { return (K + 31) / 32; }
 inline long long gs_sieve_ws_bytes(long long K) { return gs_sieve_tiles(K) * (3 * 64 * 16 + 16) + 16; }
 
 __global__ __launch_bounds__(128) void k_sieve_pack(const double* __restrict__ ubis, int K,
                                                     gs_half8* __restrict__ frag,
                                                     float* __restrict__ span,
-                                                    int* __restrict__ counts) {
+                                                    int* __restrict__ counts, int copies) {
     __shared__ float lspan[96];
     const int tl = blockIdx.x, t = threadIdx.x;
-    if (t < 32 && 32 * tl + t < K) counts[32 * tl + t] = 0;
+    if (32 * tl + (t & 31) < K)
+        for (int c = t / 32; c < copies; c += 4) counts[(size_t)c * K + 32 * tl + (t & 31)] = 0;
     if (t < 96) {  // one grain row each
         const int row = t / 32, col = t & 31;
         const int g = min(32 * tl + col, K - 1);
@@ -223,7 +249,8 @@ template <bool SELECT>
 __global__ __launch_bounds__(GS_BLOCK, 4) void k_score_mfma(
     const double* __restrict__ ubis, int K, int tsplit, int nsplit, const double* __restrict__ gv,
     int ng, double tolsq, const gs_half8* __restrict__ frag, const float* __restrict__ span,
-    int* __restrict__ counts, const long long* __restrict__ off, int* __restrict__ idx) {
+    int* __restrict__ priv, int copies, const long long* __restrict__ off, int* __restrict__ idx) {
+    int* counts = priv + (size_t)(blockIdx.x % copies) * K;
     constexpr int NW = GS_BLOCK / GS_WAVE;
     constexpr int NB = GS_SIEVE_SETS;
     static_assert(8 * NB <= 32, "a queue entry holds 5 bits of quad");

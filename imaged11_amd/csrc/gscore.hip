@@ -31,6 +31,7 @@
 #include "gs_assign_gv.h"
 #include "gs_assign_mfma.h"
 #include "gs_index.h"
+#include "gs_lists.h"
 #include "gs_geometry.h"
 #include "gs_grains.h"
 #include "gs_pbp.h"
@@ -326,11 +327,21 @@ int launch_sieve(const double* ubis, int K, const double* gv, int ng, double tol
     const int tiles = (int)gs_sieve_tiles(K);
     gs_half8* frag = static_cast<gs_half8*>(ws);
     float* span = reinterpret_cast<float*>(frag + 3 * (size_t)tiles * GS_WAVE);
-    hipLaunchKernelGGL(k_sieve_pack, dim3(tiles), dim3(128), 0, st, ubis, K, frag, span, counts);
+    // few grains: the blocks' counts meet on few addresses (gs_copies)
+    const int copies = !SELECT && K <= GS_SCORE_COPIES_MAX ? gs_copies(K) : 1;
+    int* into = copies > 1 ? reinterpret_cast<int*>(static_cast<char*>(ws) + gs_sieve_ws_bytes(K))
+                           : counts;
+    hipLaunchKernelGGL(k_sieve_pack, dim3(tiles), dim3(128), 0, st, ubis, K, frag, span, into,
+                       copies);
     GS_LAUNCHED();
     hipLaunchKernelGGL(k_score_mfma<SELECT>, dim3(nb), dim3(GS_BLOCK), 0, st, ubis, K, tsplit,
-                       nsplit, gv, ng, tolsq, frag, span, counts, off, idx);
+                       nsplit, gv, ng, tolsq, frag, span, into, copies, off, idx);
     GS_LAUNCHED();
+    if (copies > 1) {
+        hipLaunchKernelGGL(k_sum_copies, dim3(blocks_for(K, GS_BLOCK)), dim3(GS_BLOCK), 0, st, into,
+                           copies, K, counts);
+        GS_LAUNCHED();
+    }
     return GS_OK;
 }
 
@@ -413,10 +424,11 @@ template <bool GEOM, int NB>
 int launch_assign_nb(const double* gvx, const double* so, const double* co, int ng,
                      const gs_goniometer& gp, const double* ubis, const double* trans, int K,
                      double tolsq, const gs_half8* frag, const gs_tile_info* info,
-                     const int* yexp, double* drlv2, int* labels, int* counts, hipStream_t st) {
+                     const int* yexp, double* drlv2, int* labels, int* priv, int copies,
+                     hipStream_t st) {
     const int nb = blocks_for(ng, 32 * NB * (GS_BLOCK / GS_WAVE));
     hipLaunchKernelGGL((k_assign_mfma<GEOM, NB>), dim3(nb), dim3(GS_BLOCK), 0, st, gvx, so, co, ng,
-                       gp, ubis, trans, K, tolsq, frag, info, yexp, drlv2, labels, counts);
+                       gp, ubis, trans, K, tolsq, frag, info, yexp, drlv2, labels, priv, copies);
     GS_LAUNCHED();
     return GS_OK;
 }
@@ -437,18 +449,21 @@ int launch_assign_sieve(const double* gvx, const double* so, const double* co, i
     gs_half8* frag = static_cast<gs_half8*>(ws);
     gs_tile_info* info = reinterpret_cast<gs_tile_info*>(frag + 3 * (size_t)tiles * GS_WAVE);
     int* yexp = reinterpret_cast<int*>(info + tiles);
+    int* priv = yexp + 4;
+    const int copies = gs_copies(K);
     hipLaunchKernelGGL(k_assign_pack<GEOM>, dim3(tiles), dim3(128), 0, st, ubis, trans, K, frag,
-                       info, yexp, counts);
+                       info, yexp, priv, copies);
     GS_LAUNCHED();
     const long long waves = 8LL * ctx->cus;
-    if (ng >= 128 * waves)
-        return launch_assign_nb<GEOM, 4>(gvx, so, co, ng, gp, ubis, trans, K, tol * tol, frag, info,
-                                         yexp, drlv2, labels, counts, st);
-    if (ng >= 64 * waves)
-        return launch_assign_nb<GEOM, 2>(gvx, so, co, ng, gp, ubis, trans, K, tol * tol, frag, info,
-                                         yexp, drlv2, labels, counts, st);
-    return launch_assign_nb<GEOM, 1>(gvx, so, co, ng, gp, ubis, trans, K, tol * tol, frag, info,
-                                     yexp, drlv2, labels, counts, st);
+    const auto pairs = ng >= 128 * waves  ? launch_assign_nb<GEOM, 4>
+                       : ng >= 64 * waves ? launch_assign_nb<GEOM, 2>
+                                          : launch_assign_nb<GEOM, 1>;
+    GS_CHECK(pairs(gvx, so, co, ng, gp, ubis, trans, K, tol * tol, frag, info, yexp, drlv2, labels,
+                   priv, copies, st));
+    hipLaunchKernelGGL(k_sum_copies, dim3(blocks_for(K, GS_BLOCK)), dim3(GS_BLOCK), 0, st, priv,
+                       copies, K, counts);
+    GS_LAUNCHED();
+    return GS_OK;
 }
 
 // Blocks of the one-grain refinement: one per 4·GS_BLOCK peaks, at most
@@ -1109,7 +1124,14 @@ int gs_score_many(const double* ubis, int K, const double* gv, int ng, double to
     return launch_score_many(ubis, K, gv, ng, tol, counts, peaks_per_lane, mode, S(stream));
 }
 
-long long gs_sieve_workspace_bytes(int K) { return gs_sieve_ws_bytes(K > 0 ? K : 0); }
+long long gs_sieve_workspace_bytes(int K) {
+    if (K <= 0) return 0;
+    return gs_sieve_ws_bytes(K) + (K <= GS_SCORE_COPIES_MAX ? 4LL * gs_copies(K) * K : 0);
+}
+
+long long gs_assign_workspace_bytes(int K) {
+    return K > 0 ? gs_sieve_ws_bytes(K) + 4LL * gs_copies(K) * K : 0;
+}
 
 int gs_score_many_ws(const double* ubis, int K, const double* gv, int ng, double tol, int* counts,
                      void* ws, gs_stream_t stream) {
@@ -1638,6 +1660,85 @@ int gs_gv_assign_many_ws(const double* xlylzl, const double* so, const double* c
     return launch_assign_sieve<true>(xlylzl, so, co, ng,
                                      make_gonio(1.0, wvln, wedge, chi, nullptr, mat), ubis, trans,
                                      K, tol, drlv2, labels, counts, ws, S(stream));
+}
+
+// ---- peak lists from labels --------------------------------------------------
+
+// Whether the label kernels count in LDS first, and their blocks: with 8
+// peaks per label and block or more the block's atomics are fewer than its
+// peaks; below that the labels hardly collide.
+static bool list_local(const DeviceCtx* ctx, int n, int K, int* nb) {
+    const long long blocks = (long long)n / (8LL * K);
+    const bool local = K <= GS_LIST_LOCAL && blocks >= 1;
+    const int most = blocks_for(n, 1024);
+    *nb = std::min(most, local ? (int)std::min<long long>(std::max<long long>(blocks, 8), 2 * ctx->cus)
+                               : 2 * ctx->cus);
+    return local;
+}
+
+int gs_label_counts(const int* labels, int n, int K, int* counts, gs_stream_t stream) {
+    DeviceCtx* ctx;
+    GS_CHECK(get_ctx(&ctx));
+    if (K < 0 || n < 0) return set_err(GS_ERR_ARG, "gs_label_counts: negative size");
+    GS_CHECK(fill_i32(counts, 0, K, S(stream)));
+    if (K == 0 || n == 0) return GS_OK;
+    int nb;
+    if (list_local(ctx, n, K, &nb))
+        hipLaunchKernelGGL(k_label_counts<true>, dim3(nb), dim3(1024), K * sizeof(int), S(stream),
+                           labels, n, K, counts);
+    else
+        hipLaunchKernelGGL(k_label_counts<false>, dim3(nb), dim3(1024), 0, S(stream), labels, n, K,
+                           counts);
+    GS_LAUNCHED();
+    return GS_OK;
+}
+
+int gs_list_offsets(const int* counts, int K, long long* off, int* cursor, long long* info,
+                    gs_stream_t stream) {
+    DeviceCtx* ctx;
+    GS_CHECK(get_ctx(&ctx));
+    if (K < 0) return set_err(GS_ERR_ARG, "gs_list_offsets: negative K");
+    hipLaunchKernelGGL(k_list_offsets, dim3(1), dim3(GS_SCAN_THREADS), 0, S(stream), counts, K, off,
+                       cursor, info);
+    GS_LAUNCHED();
+    return GS_OK;
+}
+
+int gs_list_fill(const int* labels, int n, int K, const long long* off, int* cursor,
+                 long long longest, int* idx, int* owner, gs_stream_t stream) {
+    DeviceCtx* ctx;
+    GS_CHECK(get_ctx(&ctx));
+    if (K < 0 || n < 0) return set_err(GS_ERR_ARG, "gs_list_fill: negative size");
+    if (longest < 0 || longest > GS_LIST_SORT_MAX)
+        return set_err(GS_ERR_ARG, "gs_list_fill: a list of %lld entries (at most %d)", longest,
+                       GS_LIST_SORT_MAX);
+    if (K == 0 || n == 0 || longest == 0) return GS_OK;
+    int nb;
+    if (list_local(ctx, n, K, &nb))
+        hipLaunchKernelGGL(k_list_fill<true>, dim3(nb), dim3(1024), K * sizeof(int), S(stream),
+                           labels, n, K, off, cursor, idx);
+    else
+        hipLaunchKernelGGL(k_list_fill<false>, dim3(nb), dim3(1024), 0, S(stream), labels, n, K, off,
+                           cursor, idx);
+    GS_LAUNCHED();
+    size_t p = 1;
+    while (p < (size_t)longest) p <<= 1;
+    hipLaunchKernelGGL(k_list_sort, dim3(K), dim3(GS_BLOCK), p * sizeof(int), S(stream), idx, off,
+                       owner);
+    GS_LAUNCHED();
+    return GS_OK;
+}
+
+int gs_list_order(const long long* off, int K, int* order, gs_stream_t stream) {
+    DeviceCtx* ctx;
+    GS_CHECK(get_ctx(&ctx));
+    if (K < 0 || K > GS_ORDER_MAX)
+        return set_err(GS_ERR_ARG, "gs_list_order: %d grains (0 to %d)", K, GS_ORDER_MAX);
+    if (K == 0) return GS_OK;
+    hipLaunchKernelGGL(k_list_order, dim3(blocks_for(K, GS_BLOCK / GS_WAVE)), dim3(GS_BLOCK), 0,
+                       S(stream), off, K, order);
+    GS_LAUNCHED();
+    return GS_OK;
 }
 
 int gs_gv_lists(const double* xlylzl, const double* so, const double* co, int ng, double wvln,

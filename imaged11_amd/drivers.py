@@ -47,10 +47,7 @@ def fight_over_peaks(ubis, gv, hkl_tol):
     drlv2 = torch.full((N,), 2.0, dtype=torch.float64, device=gv.device)
     labels = torch.full((N,), -1, dtype=torch.int32, device=gv.device)
     batched.assign_many(ubis, gv, hkl_tol, drlv2, labels)
-    K = ubis.shape[0]
-    lab = labels.long()
-    gas = torch.bincount(lab[lab >= 0], minlength=K)[:K].to(torch.int32)
-    return labels, drlv2, gas
+    return labels, drlv2, batched.label_counts(labels, ubis.shape[0])
 
 
 def getind(ubi, gv, tol):

@@ -151,7 +151,9 @@ int gs_assign_many(const double *ubis, const int *grain_labels, int K, const dou
 
 /* The same with label g for grain g (grain_labels = 0..K-1) and the sieve on
  * the matrix cores in front (same results at any tol; its fastest form for
- * |tol| <= 0.1).  ws as for gs_score_many_ws; K <= 2^24. */
+ * |tol| <= 0.1).  ws as for gs_score_many_ws, of gs_assign_workspace_bytes(K)
+ * bytes; K <= 2^24. */
+long long gs_assign_workspace_bytes(int K);
 int gs_assign_many_ws(const double *ubis, int K, const double *gv, int ng, double tol,
                       double *drlv2, int *labels, int *counts, void *ws, gs_stream_t stream);
 
@@ -384,6 +386,21 @@ int gs_gv_assign_many_ws(const double *xlylzl, const double *so, const double *c
                          double wvln, double wedge, double chi, const double *mat,
                          const double *ubis, const double *trans, int K, double tol,
                          double *drlv2, int *labels, int *counts, void *ws, gs_stream_t stream);
+
+/* Peak lists of labels 0..K-1 (other labels belong to none), peaks ascending
+ * in each, in three calls.  counts (K) and cursor (K) int32, off (K+1) int64,
+ * info[2] = {entries of all lists, entries of the longest} on the device;
+ * after reading info the caller provides idx and owner (info[0] int32 each)
+ * and passes info[1] as longest (at most 16384). */
+int gs_label_counts(const int *labels, int n, int K, int *counts, gs_stream_t stream);
+int gs_list_offsets(const int *counts, int K, long long *off, int *cursor, long long *info,
+                    gs_stream_t stream);
+int gs_list_fill(const int *labels, int n, int K, const long long *off, int *cursor,
+                 long long longest, int *idx, int *owner, gs_stream_t stream);
+/* order (K): the grains by falling list length, equal ones in grain order
+ * (what gs_refine_lists takes); K at most 8192. */
+int gs_list_order(const long long *off, int K, int *order, gs_stream_t stream);
+
 
 
 /* out[q] = compute_gv of peak idx[q] for the translation of grain owner[q]

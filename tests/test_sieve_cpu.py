@@ -48,12 +48,6 @@ def test_sieve_error_bound(mode, span, start, err):
     assert worst > err / 200  # the test reaches the range the bound is for
 
 
-def test_workspace_size_is_the_library_s():
-    from imaged11_amd import _lib
-    for K in (0, 1, 31, 32, 33, 1000, 20000):
-        assert _lib.sieve_ws(K, "cpu").numel() == _lib.load().gs_sieve_workspace_bytes(K)
-
-
 @pytest.mark.parametrize("ratio", [1e-4, 2e-3, 0.03, 0.1, 0.2])
 def test_position_expansion_error_bound(ratio):
     """u.G for a grain at t against the sieve's terms: G0 and the products p q
