@@ -2119,6 +2119,12 @@ int gs_orient_hits(const double* gv, int ng, const int* hi, const int* hj, int n
     return GS_OK;
 }
 
+int gs_select_many_ws(const double* ubis, int K, const double* gv, int ng, double thr,
+                      const long long* off, int* cursor, int* idx, void* ws, gs_stream_t stream) {
+    if (idx && !off) return set_err(GS_ERR_ARG, "gs_select_many_ws: idx needs off");
+    return launch_sieve<true>(ubis, K, gv, ng, thr, cursor, off, idx, ws, S(stream));
+}
+
 int gs_select_many(const double* ubis, int K, const double* gv, int ng, double thr,
                    const long long* off, int* cursor, int* idx, gs_stream_t stream) {
     DeviceCtx* ctx;

@@ -230,13 +230,27 @@ def select_lists(ubis, gv, thr, counts=None, sort=True):
     K, N = ubis.shape[0], gv.shape[0]
     cnt = torch.empty(K, dtype=torch.int32, device=dev)
 
+    # few pairs pass at small thr: the matrix-core sieve, where it pays
+    ws = None
+    if thr <= _lib.SIEVE_TOL_MAX ** 2 and batched.mfma_pays(K, N):
+        ws = _lib.sieve_ws(K, dev)
+
+    def select(off, idx):
+        off, idx = (None if a is None else dptr(a) for a in (off, idx))
+        if ws is not None:
+            _lib.check(lib.gs_select_many_ws(dptr(ubis), K, dptr(gv), N, float(thr), off,
+                                             dptr(cnt), idx, dptr(ws), stream_ptr()),
+                       "select_many")
+        else:
+            _lib.check(lib.gs_select_many(dptr(ubis), K, dptr(gv), N, float(thr), off, dptr(cnt),
+                                          idx, stream_ptr()), "select_many")
+
     def fill(off, total, count=False):
         # count=True: the pass also gives the counts (cnt), so it runs
         # even when there is no room at all
         idx = torch.empty(max(total, 1), dtype=torch.int32, device=dev)
         if total or count:
-            _lib.check(lib.gs_select_many(dptr(ubis), K, dptr(gv), N, float(thr), dptr(off),
-                                          dptr(cnt), dptr(idx), stream_ptr()), "select_many")
+            select(off, idx)
         return idx
 
     def offsets(c):
@@ -266,8 +280,7 @@ def select_lists(ubis, gv, thr, counts=None, sort=True):
             off, total = offsets(got)
             idx = fill(off, total)
     else:
-        _lib.check(lib.gs_select_many(dptr(ubis), K, dptr(gv), N, float(thr), None, dptr(cnt),
-                                      None, stream_ptr()), "select_many")
+        select(None, None)
         off = torch.zeros(K + 1, dtype=torch.int64, device=dev)
         torch.cumsum(cnt.to(torch.int64), 0, out=off[1:])
         total = int(off[-1].item())

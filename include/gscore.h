@@ -621,6 +621,10 @@ int gs_orient_hits(const double *gv, int ng, const int *hi, const int *hj, int n
  * thr <= 0.01 the one-row sieve of GS_SCORE_SIEVE runs first. */
 int gs_select_many(const double *ubis, int K, const double *gv, int ng, double thr,
                    const long long *off, int *cursor, int *idx, gs_stream_t stream);
+/* The same behind the matrix-core sieve; ws as for gs_score_many_ws. */
+int gs_select_many_ws(const double *ubis, int K, const double *gv, int ng, double thr,
+                      const long long *off, int *cursor, int *idx, void *ws,
+                      gs_stream_t stream);
 
 /* One iteration of B Nelder-Mead simplexes of n <= 64 variables stepped in
  * lockstep, on HOST arrays, split where the objective is called

@@ -216,3 +216,30 @@ def test_assignment_over_the_ranges_of_the_accumulator(dev, orc, cell, gmax):
     assert want.sum() > 0 and np.array_equal(got.cpu().numpy(), want)
     assert np.array_equal(ll.cpu().numpy(), lab)
     assert np.array_equal(dd.cpu().numpy().view(np.int64), d.view(np.int64))
+
+
+@pytest.mark.parametrize("K,N", [(8, 2000003), (700, 30001), (2100, 8000)])
+@pytest.mark.parametrize("tol", [0.02, 0.1])
+def test_selected_lists(dev, K, N, tol):
+    """select_lists at the sizes that take the sieve, in one pass (exact and
+    too small room) and in two, against the reference arithmetic."""
+    from imaged11_amd import indexing
+    assert batched.mfma_pays(K, N)
+    ubi, gv = make(K, N, N)
+    u, g = T(ubi, dev), T(gv, dev)
+    thr = tol * tol
+    n = batched.score_many(u, g, tol, exact=True).cpu().numpy()
+    want = []
+    for k in range(0, K, max(1, K // 5)):
+        h = gv @ ubi[k].T
+        d = ((h - np.rint(h)) ** 2).sum(1)
+        edge = np.abs(d - thr) < 1e-12
+        want.append((k, np.nonzero(d < thr)[0], edge.any()))
+    for counts in (None, n, np.maximum(n // 2, 1), n + 5):
+        idx, off = indexing.select_lists(u, g, thr, counts=counts)
+        idx, off = idx.cpu().numpy(), off.cpu().numpy()
+        assert np.array_equal(np.diff(off), n)
+        for k, w, edge in want:
+            got = idx[off[k]:off[k + 1]]
+            assert np.all(np.diff(got) > 0)
+            assert edge or np.array_equal(got, w)
