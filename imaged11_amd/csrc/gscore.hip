@@ -1882,7 +1882,7 @@ int gs_pbp_ubi_fit(const double* design, const long long* off, const int* fit,
     if (!B0) return set_err(GS_ERR_ARG, "gs_pbp_ubi_fit: null B0");
     gs_mat9 b;
     for (int i = 0; i < 9; i++) b.m[i] = B0[i];
-    hipLaunchKernelGGL(k_pbp_ubi_fit, dim3(blocks_for(T, 64)), dim3(64), 0, S(stream), design, off,
+    hipLaunchKernelGGL(k_pbp_ubi_fit, dim3(blocks_for(T, 64 / GS_FIT_LANES)), dim3(64), 0, S(stream), design, off,
                        fit, ubi_in, b, T, ubifit, rank, worth, ubi_out, ub0);
     GS_LAUNCHED();
     return GS_OK;
@@ -1894,7 +1894,7 @@ int gs_pbp_strain_fit(const double* design, const long long* off, const int* wor
     GS_CHECK(get_ctx(&ctx));
     if (T < 0) return set_err(GS_ERR_ARG, "gs_pbp_strain_fit: negative task count");
     if (T == 0) return GS_OK;
-    hipLaunchKernelGGL(k_pbp_strain_fit, dim3(blocks_for(T, 64)), dim3(64), 0, S(stream), design,
+    hipLaunchKernelGGL(k_pbp_strain_fit, dim3(blocks_for(T, 64 / GS_FIT_LANES)), dim3(64), 0, S(stream), design,
                        off, worth, T, eps);
     GS_LAUNCHED();
     return GS_OK;
