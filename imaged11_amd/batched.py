@@ -38,13 +38,25 @@ def _ready():
 from ._lib import SIEVE_TOL_MAX, score_mode  # noqa: E402  (the default score kernel)
 
 
+MFMA_PAIRS = 16000000  # the least pairs for which the matrix cores pay
+
+
 def mfma_pays(K, N):
     """Whether the matrix-core sieve is the faster one for K grains x N
     peaks.  Its tiles hold 32 grains (4 x 10^6: 20 us against 18 of the row
     sieve, 16 x 10^6: 20 against 31), and its workspace and launches cost the
     host 1.5 to 4 us a call, which is all there is to a small problem (300 x
     30 000: 18 us against 14, 1000 x 30 000: 17 against 23)."""
-    return K >= 8 and K * N >= 16000000
+    return K >= 8 and K * N >= MFMA_PAIRS
+
+
+def ball_pays(K, N, tol):
+    """Whether the matrix cores pay beyond the sieves' tolerances, where the
+    ball counts the pairs (gs_ball_tile): 257 x 300007 at tol 0.25 40 us
+    against 59 of the all-rows kernel, 1000 x 10^6 290 against 611, 16 x 10^6
+    26 against 30; 100 x 160000 took 20 against 18 and 8 x 2 10^6 41 against
+    31.  From 0.75 on nearly every pair counts and no caller asks."""
+    return K * N >= 32000000 and K >= 16 and _lib.SIEVE_TOL_MAX < abs(float(tol)) < 0.75
 
 
 def assign_mfma_pays(K, N, tol):
@@ -57,8 +69,8 @@ def assign_mfma_pays(K, N, tol):
 
 
 def score_sieve(ubis, gv, tol, out=None):
-    """score_many by the sieve on the matrix cores (gs_score_many_ws), at any
-    size and tolerance."""
+    """score_many on the matrix cores (gs_score_many_ws), at any size and
+    tolerance."""
     lib = _ready()
     _need(ubis, torch.float64, "ubis", (None, 3, 3))
     _need(gv, torch.float64, "gv", (None, 3))
@@ -78,20 +90,26 @@ def score_many(ubis, gv, tol, peaks_per_lane=0, out=None, exact=False, mode=None
     ubis (K,3,3) float64, gv (N,3) float64 -> int32 (K,).  exact=True uses
     the reference's arithmetic for every pair; by default the certified
     kernel score_mode(tol) picks runs; every mode returns the reference's
-    counts.  Of the two sieves, mfma_pays(K, N) picks (a tile height
-    peaks_per_lane asks for the row sieve on the vector ALU)."""
+    counts.  mfma_pays and ball_pays say when the matrix cores take the
+    call instead (a tile height peaks_per_lane asks for the kernels on the
+    vector ALU, and so does mode=SCORE_CERTIFIED)."""
     lib = _ready()
     _need(ubis, torch.float64, "ubis", (None, 3, 3))
     _need(gv, torch.float64, "gv", (None, 3))
-    K = ubis.shape[0]
+    K, N = ubis.shape[0], gv.shape[0]
     if out is None:
         out = torch.empty(K, dtype=torch.int32, device=gv.device)
     _need(out, torch.int32, "out", (K,))
     if mode is None:
         mode = _lib.SCORE_EXACT if exact else score_mode(tol)
-    if mode == _lib.SCORE_SIEVE and not peaks_per_lane and mfma_pays(K, gv.shape[0]):
+        ball = not exact
+    else:
+        ball = False
+    # (the pairs first: a small problem's time is this host code)
+    if K * N >= MFMA_PAIRS and not peaks_per_lane and (
+            mode == _lib.SCORE_SIEVE and mfma_pays(K, N) or ball and ball_pays(K, N, tol)):
         return score_sieve(ubis, gv, tol, out)
-    _lib.check(lib.gs_score_many(dptr(ubis), K, dptr(gv), gv.shape[0], float(tol), dptr(out),
+    _lib.check(lib.gs_score_many(dptr(ubis), K, dptr(gv), N, float(tol), dptr(out),
                                  int(peaks_per_lane), mode, stream_ptr()), "score_many")
     return out
 

@@ -50,6 +50,7 @@
 
 typedef _Float16 gs_half8 __attribute__((ext_vector_type(8)));
 typedef float gs_float16 __attribute__((ext_vector_type(16)));
+typedef short gs_short2 __attribute__((ext_vector_type(2)));
 
 #define GS_SIEVE_SPAN 60.0f
 #define GS_SIEVE_SPAN_WIDE 1000.0f
@@ -57,6 +58,11 @@ typedef float gs_float16 __attribute__((ext_vector_type(16)));
 #define GS_SIEVE_GMAX 30.0f
 #define GS_SIEVE_ERR 0x1p-11
 #define GS_SIEVE_ERR_WIDE 0x1p-7
+// The ball (gs_ball_tile) is the faster one from here (1000 x 10^6 at tol 0.1:
+// sieve 207 us, ball 282; at 0.2 a quarter of all quads would pass the sieve),
+// up to where a dead pair's S, 3/4, could come near the tolerance.
+#define GS_BALL_TOL_MIN 0.1
+#define GS_BALL_TOL_MAX 0.75
 #define GS_SIEVE_SETS 4    // 32-peak sets per wave (NB)
 #define GS_SIEVE_SPLIT 64  // grain tiles of a block's split at most (its counters in LDS)
 
@@ -76,6 +82,16 @@ GS_HD __forceinline__ void gs_sieve_units(double r, int& r16, int& thr) {
         r16 = 0;
         thr = 0xffff;
     }
+}
+
+// the bounds of gs_ball_tile for tolerance tol and an error err per row, one
+// unit of S outward each: lo = 2^32 (tol - sqrt(3) err)^2 (0: nothing is
+// certain), lo + width = 2^32 (tol + sqrt(3) err)^2
+GS_HD __forceinline__ void gs_ball_units(double tol, double err, unsigned& lo, unsigned& width) {
+    const double e = 1.7320508075688774 * err + 1e-9;
+    const double a = fmax(tol - e, 0.0) * 65536.0, b = (tol + e) * 65536.0;
+    lo = (unsigned)fmax(a * a - 1.0, 0.0);
+    width = (unsigned)(b * b + 2.0) - lo;
 }
 
 // A peak's 16 k slots, the half this lane holds (k = 8 half + j); p may be
@@ -165,6 +181,63 @@ __device__ __forceinline__ void gs_sieve_tile(gs_half8 pk, gs_half8 b0, gs_half8
     }
 }
 
+// The same tile by the ball: with the accumulator started at 1.5 2^23 itself
+// its low 16 bits, signed, are 2^16 (h - round(h)), and S, the sum of their
+// three squares (at most 3 2^30, so it wraps nowhere as an unsigned number),
+// is 2^32 drlv2 with each root off by GS_SIEVE_ERR at most.  By the triangle
+// inequality S < lo counts for certain and S >= lo + width does not (lo,
+// width of gs_ball_units); only a quad with a pair between them is queued.
+// Returns how many pairs of the lane's grain count in the quads not queued.
+// 11 vector instructions of 32 bits or less per pair (a byte permute, two
+// 16-bit dot products, a mask, and the subtraction, carry and minimum of the
+// two tests) against 14 of FP64 in k_score_many_fast.  Bound by their issue:
+// 1000 grains x 10^6 peaks at tol 0.25 290 us against 611, 257 x 300007 40
+// against 59.
+template <bool WIDE, class Entry>
+__device__ __forceinline__ int gs_ball_tile(gs_half8 pk, gs_half8 b0, gs_half8 b1, gs_half8 b2,
+                                            gs_float16 c, unsigned lo, unsigned width, unsigned lp,
+                                            Entry* q, int& qn) {
+    const gs_float16 h0 = __builtin_amdgcn_mfma_f32_32x32x16_f16(pk, b0, c, 0, 0, 0);
+    const gs_float16 h1 = __builtin_amdgcn_mfma_f32_32x32x16_f16(pk, b1, c, 0, 0, 0);
+    const gs_float16 h2 = __builtin_amdgcn_mfma_f32_32x32x16_f16(pk, b2, c, 0, 0, 0);
+    int n = 0;
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        unsigned w = 0xffffffffu;
+        int n4 = 0;
+#pragma unroll
+        for (int i = 4 * j; i < 4 * j + 4; i++) {
+            unsigned x = __builtin_bit_cast(unsigned, (float)h0[i]);
+            unsigned y = __builtin_bit_cast(unsigned, (float)h1[i]);
+            unsigned z = __builtin_bit_cast(unsigned, (float)h2[i]);
+            if (WIDE) {
+                x <<= 4;
+                y <<= 4;
+                z <<= 4;
+            }
+            const gs_short2 xy = __builtin_bit_cast(gs_short2, __builtin_amdgcn_perm(y, x, 0x05040100u));
+            const gs_short2 z0 = __builtin_bit_cast(gs_short2, z & 0xffffu);
+            const unsigned S = (unsigned)__builtin_amdgcn_sdot2(
+                xy, xy, __builtin_amdgcn_sdot2(z0, z0, 0, false), false);
+            n4 += S < lo;
+            w = min(w, S - lo);
+        }
+        const bool in = w < width;
+        const unsigned long long m = __builtin_amdgcn_ballot_w64(in);
+        if (m) {
+            if (in) {
+                const unsigned pos = __builtin_amdgcn_mbcnt_hi(
+                    (unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u));
+                (q + qn)[pos] = (Entry)(lp + 2 * j);
+                n4 = 0;
+            }
+            qn += __popcll(m);
+        }
+        n += n4;
+    }
+    return n;
+}
+
 __device__ __forceinline__ gs_float16 gs_splat16(float v) {
     return (gs_float16){v, v, v, v, v, v, v, v, v, v, v, v, v, v, v, v};
 }
@@ -196,7 +269,9 @@ __global__ __launch_bounds__(GS_BLOCK) void k_sum_copies(const int* __restrict__
 
 // ---------------------------------------------------------------------------
 // The grains' fragments, packed once per call into the caller's workspace:
-// tile t (grains 32 t .. 32 t + 31; past K the last grain again) has
+// tile t (grains 32 t .. 32 t + 31; "dead" past K and where u is not finite,
+// as a peak is past the list and where g is not finite: zeros, and 1/2 of h
+// from the p, q slots, which passes no sieve and no ball) has
 // 3 x 64 x 16 bytes, row-major by UBI row, lane l holding column l & 31 and k
 // slots 8 (l >> 5) .. + 7, then one float per tile, the largest row sum of
 // |u|.  Also clears the counters (so that no separate fill is launched).
@@ -213,18 +288,20 @@ __global__ __launch_bounds__(128) void k_sieve_pack(const double* __restrict__ u
         for (int c = t / 32; c < copies; c += 4) counts[(size_t)c * K + 32 * tl + (t & 31)] = 0;
     if (t < 96) {  // one grain row each
         const int row = t / 32, col = t & 31;
-        const int g = min(32 * tl + col, K - 1);
-        const double* u = ubis + 9 * (size_t)g + 3 * row;
+        const int g = 32 * tl + col;
+        const double* u = ubis + 9 * (size_t)min(g, K - 1) + 3 * row;
         double u0 = u[0], u1 = u[1], u2 = u[2];
         float a = (float)(fabs(u0) + fabs(u1) + fabs(u2));
-        if (!(a < __builtin_inff())) {  // never counted, whatever it passes
+        const bool live = g < K && gs_finite(u0) && gs_finite(u1) && gs_finite(u2);
+        if (!live) {
             u0 = u1 = u2 = 0.0;
             a = 0.0f;
         }
+        const double q[7] = {live ? 1.0 : 0.0, live ? 0.0 : 32768.0, 0.0, 0.0, 0.0, 0.0, 0.0};
         lspan[t] = a * (1.0f + 0x1p-20f);
         gs_half8* f = frag + (3 * (size_t)tl + row) * GS_WAVE;
         gs_half8 lo, hi;
-        gs_grain_frag(u0, u1, u2, nullptr, lo, hi);
+        gs_grain_frag(u0, u1, u2, q, lo, hi);
         f[col] = lo;
         f[col + 32] = hi;
     }
@@ -245,7 +322,8 @@ __global__ __launch_bounds__(128) void k_sieve_pack(const double* __restrict__ u
 // are settled, one quad per lane, by gs_drlv2.
 // SELECT: cursor = counts; a pair that counts takes a slot of its grain and,
 // when idx is given, writes its peak number there (see k_select_many).
-template <bool SELECT>
+// BALL: gs_ball_tile in the place of the sieve.
+template <bool SELECT, bool BALL>
 __global__ __launch_bounds__(GS_BLOCK, 4) void k_score_mfma(
     const double* __restrict__ ubis, int K, int tsplit, int nsplit, const double* __restrict__ gv,
     int ng, double tolsq, const gs_half8* __restrict__ frag, const float* __restrict__ span,
@@ -268,20 +346,19 @@ __global__ __launch_bounds__(GS_BLOCK, 4) void k_score_mfma(
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / GS_WAVE);
     const int half = lane >> 5;
     for (int i = threadIdx.x; i < 32 * (t1 - t0); i += GS_BLOCK) lcnt[i] = 0;
-    // this wave's peaks: k0 .. k0 + 32 NB - 1, those past ng repeat the last
+    // this wave's peaks: k0 .. k0 + 32 NB - 1
     const long long k0 = (long long)chunk * (NW * NB * 32) + wave * (NB * 32);
     float gmax = 0.0f;
     for (int s = 0; s < NB; s++) {
         long long k = k0 + 32 * s + (lane & 31);
-        k = k < ng ? k : (long long)ng - 1;
+        bool live = k < ng;
+        k = live ? k : (long long)ng - 1;
         double x = gv[3 * k], y = gv[3 * k + 1], z = gv[3 * k + 2];
-        if (!(gs_finite(x) && gs_finite(y) && gs_finite(z))) {
-            x = 0.3137;  // a NaN drlv2 in any case: never counted
-            y = 0.2711;
-            z = 0.1873;
-        }
+        live = live && gs_finite(x) && gs_finite(y) && gs_finite(z);
+        if (!live) x = y = z = 0.0;
+        const double p[7] = {live ? 0.0 : 32768.0, 1.0, 0.0, 0.0, 0.0, 0.0, 0.0};
         gmax = fmaxf(gmax, (float)fmax(fabs(x), fmax(fabs(y), fabs(z))));
-        lpk[wave][s][lane] = gs_peak_frag(x, y, z, nullptr, half);
+        lpk[wave][s][lane] = gs_peak_frag(x, y, z, p, half);
     }
     for (int o = 1; o < 32; o <<= 1) gmax = fmaxf(gmax, __shfl_xor(gmax, o, GS_WAVE));
     gmax = __builtin_bit_cast(
@@ -290,6 +367,12 @@ __global__ __launch_bounds__(GS_BLOCK, 4) void k_score_mfma(
     int r16, thr, r16w, thrw;
     gs_sieve_units(tol + GS_SIEVE_ERR, r16, thr);
     gs_sieve_units(tol + GS_SIEVE_ERR_WIDE, r16w, thrw);
+    unsigned lo = 0, width = 0, low = 0, widthw = 0;
+    if (BALL) {
+        r16 = r16w = 0;
+        gs_ball_units(tol, GS_SIEVE_ERR, lo, width);
+        gs_ball_units(tol, GS_SIEVE_ERR_WIDE, low, widthw);
+    }
     unsigned short* q = lq[wave];
     int qn = 0;
     const auto hit = [&](int gl, long long k) {
@@ -303,12 +386,12 @@ __global__ __launch_bounds__(GS_BLOCK, 4) void k_score_mfma(
     };
     const auto settle = [&](unsigned e) {
         const int gl = e >> 5;
-        if (g0 + gl >= K) return;  // the repeated last grain
+        if (g0 + gl >= K) return;
         const gs_ubi u = gs_load_ubi(ubis + 9 * (size_t)(g0 + gl));
         const long long k = k0 + 4 * (e & 31);
 #pragma unroll
         for (int i = 0; i < 4; i++) {
-            const long long ki = min(k + i, (long long)ng - 1);  // the repeated last peak
+            const long long ki = min(k + i, (long long)ng - 1);
             if (gs_drlv2(u, gv[3 * ki], gv[3 * ki + 1], gv[3 * ki + 2]) < tolsq && k + i < ng)
                 hit(gl, k + i);
         }
@@ -337,17 +420,27 @@ __global__ __launch_bounds__(GS_BLOCK, 4) void k_score_mfma(
         }
         // entry of quad j, set s: lane part + 8 s + 2 j
         const unsigned lp = ((32 * (t - t0) + (lane & 31)) << 5) | half;
+        int n = 0;  // BALL: the certain pairs of the lane's grain
         if (fits && sp <= GS_SIEVE_SPAN) {
 #pragma unroll 1
             for (int s = 0; s < NB; s++) {
-                gs_sieve_tile<false>(lpk[wave][s][lane], b0, b1, b2, c, thr, lp + 8 * s, q, qn);
+                if constexpr (BALL)
+                    n += gs_ball_tile<false>(lpk[wave][s][lane], b0, b1, b2, c, lo, width,
+                                             lp + 8 * s, q, qn);
+                else
+                    gs_sieve_tile<false>(lpk[wave][s][lane], b0, b1, b2, c, thr, lp + 8 * s, q, qn);
                 drain();
             }
         } else if (fits && sp <= GS_SIEVE_SPAN_WIDE) {
             const gs_float16 cw = gs_splat16(201326592.0f + r16w);  // 1.5 2^27
 #pragma unroll 1
             for (int s = 0; s < NB; s++) {
-                gs_sieve_tile<true>(lpk[wave][s][lane], b0, b1, b2, cw, thrw, lp + 8 * s, q, qn);
+                if constexpr (BALL)
+                    n += gs_ball_tile<true>(lpk[wave][s][lane], b0, b1, b2, cw, low, widthw,
+                                            lp + 8 * s, q, qn);
+                else
+                    gs_sieve_tile<true>(lpk[wave][s][lane], b0, b1, b2, cw, thrw, lp + 8 * s, q,
+                                        qn);
                 drain();
             }
         } else {
@@ -360,6 +453,7 @@ __global__ __launch_bounds__(GS_BLOCK, 4) void k_score_mfma(
                 }
             }
         }
+        if (BALL && n) atomicAdd(&lcnt[32 * (t - t0) + (lane & 31)], n);
     }
     __builtin_amdgcn_wave_barrier();
     if (lane < qn) settle(q[lane]);
@@ -367,7 +461,7 @@ __global__ __launch_bounds__(GS_BLOCK, 4) void k_score_mfma(
         __syncthreads();
         for (int i = threadIdx.x; i < 32 * (t1 - t0); i += GS_BLOCK) {
             const int c = lcnt[i];
-            if (c) atomicAdd(&counts[g0 + i], c);
+            if (c && g0 + i < K) atomicAdd(&counts[g0 + i], c);
         }
     }
 }

@@ -312,7 +312,7 @@ int sieve_grid(DeviceCtx* ctx, int K, int ng, int* tsplit_out, int* nsplit_out,
 
 // score (idx, off NULL) or list extraction (SELECT) by the matrix-core
 // sieve: the pack launch, which also clears counts, and the pairs.
-template <bool SELECT>
+template <bool SELECT, bool BALL = false>
 int launch_sieve(const double* ubis, int K, const double* gv, int ng, double tolsq, int* counts,
                  const long long* off, int* idx, void* ws, hipStream_t st) {
     DeviceCtx* ctx;
@@ -334,7 +334,7 @@ int launch_sieve(const double* ubis, int K, const double* gv, int ng, double tol
     hipLaunchKernelGGL(k_sieve_pack, dim3(tiles), dim3(128), 0, st, ubis, K, frag, span, into,
                        copies);
     GS_LAUNCHED();
-    hipLaunchKernelGGL(k_score_mfma<SELECT>, dim3(nb), dim3(GS_BLOCK), 0, st, ubis, K, tsplit,
+    hipLaunchKernelGGL((k_score_mfma<SELECT, BALL>), dim3(nb), dim3(GS_BLOCK), 0, st, ubis, K, tsplit,
                        nsplit, gv, ng, tolsq, frag, span, into, copies, off, idx);
     GS_LAUNCHED();
     if (copies > 1) {
@@ -1135,6 +1135,10 @@ long long gs_assign_workspace_bytes(int K) {
 
 int gs_score_many_ws(const double* ubis, int K, const double* gv, int ng, double tol, int* counts,
                      void* ws, gs_stream_t stream) {
+    const double a = fabs(tol);
+    if (a > GS_BALL_TOL_MIN && a < GS_BALL_TOL_MAX)
+        return launch_sieve<false, true>(ubis, K, gv, ng, tol * tol, counts, nullptr, nullptr, ws,
+                                         S(stream));
     return launch_sieve<false>(ubis, K, gv, ng, tol * tol, counts, nullptr, nullptr, ws, S(stream));
 }
 

@@ -133,8 +133,8 @@ void compute_xlylzl(double s[], double f[], double p[4], double r[9], double dis
 int gs_score_many(const double *ubis, int K, const double *gv, int ng, double tol,
                   int *counts, int peaks_per_lane, int mode, gs_stream_t stream);
 
-/* gs_score_many with the sieve on the matrix cores (its fastest form for
- * |tol| <= 0.1; the reference's counts at any tol).  ws: device memory of at
+/* gs_score_many on the matrix cores: the sieve up to |tol| = 0.1, the ball
+ * beyond (the reference's counts at any tol).  ws: device memory of at
  * least gs_sieve_workspace_bytes(K) bytes, 16-byte aligned, whose contents
  * need not be kept and may be reused by later work on the stream. */
 long long gs_sieve_workspace_bytes(int K);

@@ -4,7 +4,7 @@ import numpy as np
 import pytest
 import torch
 
-from imaged11_amd import batched, simulate
+from imaged11_amd import _lib, batched, simulate
 
 pytestmark = pytest.mark.gpu
 
@@ -243,3 +243,68 @@ def test_selected_lists(dev, K, N, tol):
             got = idx[off[k]:off[k + 1]]
             assert np.all(np.diff(got) > 0)
             assert edge or np.array_equal(got, w)
+
+
+# beyond the sieves' tolerances: the ball (tile edges, the accumulator's
+# ranges, values that are not finite, distances at the tolerance)
+@pytest.mark.parametrize("K,N", [(1, 1), (1, 5000), (31, 127), (33, 129), (65, 513), (2049, 700)])
+@pytest.mark.parametrize("tol", [0.1001, 0.25, 0.499, 0.7499, 0.7501])
+def test_ball_counts_at_tile_edges(dev, orc, K, N, tol):
+    ubi, gv = make(K, N, K + N)
+    for sign in (1, -1):
+        got = batched.score_sieve(T(ubi, dev), T(gv, dev), sign * tol)
+        assert np.array_equal(got.cpu().numpy(), orc.score_many(ubi, gv, tol))
+
+
+@pytest.mark.parametrize("cell,gmax", [((10.0, 20.0), 1.6), ((20.0, 60.0), 1.6),
+                                       ((200.0, 320.0), 1.6), ((300.0, 900.0), 1.6),
+                                       ((900.0, 2000.0), 0.01), ((1e-4, 2e-4), 1e4),
+                                       ((2e6, 5e6), 1e-6)])
+def test_ball_over_the_ranges_of_the_accumulator(dev, orc, cell, gmax):
+    ubi, gv = make(70, 3000, 5, cell=cell, gmax=gmax)
+    for tol in (0.15, 0.3):
+        got = batched.score_sieve(T(ubi, dev), T(gv, dev), tol)
+        assert np.array_equal(got.cpu().numpy(), orc.score_many(ubi, gv, tol))
+
+
+def test_ball_special_values(dev, orc):
+    ubi, gv = make(40, 1000, 11)
+    for i, v in enumerate([np.nan, np.inf, -np.inf, 1e300, 1e-310, 0.0]):
+        gv[17 * i + 3, i % 3] = v
+        gv[17 * i + 5] = v
+        ubi[2 * i, i % 3, (i + 1) % 3] = v
+        ubi[2 * i + 13] = v
+    for u, g in ((ubi, gv), (ubi[:13:2], gv), (ubi[30:], gv[200:])):
+        for tol in (0.25, 0.74):
+            got = batched.score_sieve(T(u, dev), T(g, dev), tol)
+            assert np.array_equal(got.cpu().numpy(), orc.score_many(u, g, tol))
+
+
+@pytest.mark.parametrize("tol", [0.125, 0.3, 0.49])
+def test_ball_pairs_on_the_tolerance(dev, orc, tol):
+    """Distances that straddle tol by 1e-17 .. 1e-3, along one row, two and
+    three: certain and settled pairs side by side in one quad."""
+    a, rng = 4.0, np.random.default_rng(2)
+    d = np.array([tol * (1 + s * 10.0 ** -e) for s in (-1, 1) for e in range(3, 17)])
+    gv = []
+    for axes in ((1, 0, 0), (0, -1, 0), (1, 1, 0), (1, -1, 1), (0, 2, 1)):
+        v = np.array(axes, float)
+        for h in rng.integers(-6, 7, (20, 3)):
+            gv.append((h + d[:, None] * v / np.linalg.norm(v)) / a)
+    gv = rng.permutation(np.concatenate(gv))
+    ubi = np.eye(3)[None] * a * np.array([1.0, -1.0, 1.0])[:, None, None]
+    got = batched.score_sieve(T(ubi, dev), T(gv, dev), tol).cpu().numpy()
+    want = orc.score_many(ubi, gv, tol)
+    assert 0 < want[0] < len(gv)
+    assert np.array_equal(got, want)
+
+
+@pytest.mark.parametrize("K,N", [(15, 2200000), (16, 2000000), (321, 100001)])
+def test_ball_dispatch(dev, K, N):
+    """score_many's own choice against the FP64 kernel, on both sides of the
+    rule; tol 0.74, 0.75 and 0.1 lie at its ends."""
+    ubi, gv = make(K, N, 3)
+    ubi, gv = T(ubi, dev), T(gv, dev)
+    for tol in (0.1, 0.11, 0.25, 0.74, 0.75):
+        assert torch.equal(batched.score_many(ubi, gv, tol),
+                           batched.score_many(ubi, gv, tol, mode=_lib.SCORE_CERTIFIED))
