@@ -552,8 +552,8 @@ __global__ __launch_bounds__(GS_BLOCK) void k_assign_many_fast(
 // one-block launch; ubi is then read by every thread first and written by
 // thread 0 after the block's barrier.
 __device__ __forceinline__ void gs_unpack_RH(const double* t, double* R, double* H);
-__device__ __forceinline__ void gs_refine_finish(const double* tot, double* ubi, int* n_out,
-                                                 double* mean_out);
+__device__ __forceinline__ void gs_refine_finish(const double* tot, const double* u0, double* ubi,
+                                                 int* n_out, double* mean_out);
 
 template <int MODE, bool FUSED>
 __global__ __launch_bounds__(GS_BLOCK) void k_refine_partials(
@@ -599,7 +599,10 @@ __global__ __launch_bounds__(GS_BLOCK) void k_refine_partials(
     }
     if (FUSED) {
         __syncthreads();
-        if (threadIdx.x == 0) gs_refine_finish(tot, ubi, n_out, mean_out);
+        if (threadIdx.x == 0) {
+            const double u0[9] = {u.u00, u.u01, u.u02, u.u10, u.u11, u.u12, u.u20, u.u21, u.u22};
+            gs_refine_finish(tot, u0, ubi, n_out, mean_out);
+        }
     }
 }
 
@@ -611,12 +614,13 @@ __device__ __forceinline__ void gs_unpack_RH(const double* t, double* R, double*
     H[6] = t[13]; H[7] = t[15]; H[8] = t[16];
 }
 
-// Solve from the 17 totals, UBI in place, n and the mean drlv2 (one thread).
-__device__ __forceinline__ void gs_refine_finish(const double* tot, double* ubi, int* n_out,
-                                                 double* mean_out) {
+// Solve from the 17 totals and the UBI u0, the new UBI, n and the mean drlv2
+// (one thread).
+__device__ __forceinline__ void gs_refine_finish(const double* tot, const double* u0, double* ubi,
+                                                 int* n_out, double* mean_out) {
     double R[9], H[9], u[9];
     gs_unpack_RH(tot, R, H);
-    for (int i = 0; i < 9; i++) u[i] = ubi[i];
+    for (int i = 0; i < 9; i++) u[i] = u0[i];
     gs_solve_ubi(u, R, H);
     for (int i = 0; i < 9; i++) ubi[i] = u[i];
     int n = (int)tot[0];
@@ -625,17 +629,37 @@ __device__ __forceinline__ void gs_refine_finish(const double* tot, double* ubi,
     *mean_out = n > 0 ? s / n : s;
 }
 
-__global__ void k_refine_finalize(const double* __restrict__ partials, int nblocks,
-                                  double* __restrict__ ubi, int* __restrict__ n_out,
-                                  double* __restrict__ mean_out) {
-    __shared__ double tot[GS_NPART];
-    if (threadIdx.x < GS_NPART) {
-        double v = 0.0;
-        for (int b = 0; b < nblocks; b++) v += partials[(size_t)b * GS_NPART + threadIdx.x];
-        tot[threadIdx.x] = v;
+// The blocks' partial sums in block order, one thread per quantity.  Bound by
+// latency: the partials come in through LDS, GS_FINAL_BLOCKS of them by the
+// whole block at once, and the UBI (host memory for host callers) is on its
+// way meanwhile, so the additions wait for LDS alone.  One score_and_refine
+// call with peaks on the device: 200 000 peaks (196 blocks) 79 -> 36 us, 20 000
+// (20) 35 -> 31, against each thread fetching its terms as it added them.
+#define GS_FINAL_BLOCKS 128
+__global__ __launch_bounds__(GS_BLOCK) void k_refine_finalize(
+    const double* __restrict__ partials, int nblocks, double* __restrict__ ubi,
+    int* __restrict__ n_out, double* __restrict__ mean_out) {
+    __shared__ double part[GS_FINAL_BLOCKS * GS_NPART];
+    __shared__ double tot[GS_NPART], su[9];
+    const int t = threadIdx.x;
+    if (t >= GS_BLOCK - 9) su[t - (GS_BLOCK - 9)] = ubi[t - (GS_BLOCK - 9)];
+    double v = 0.0;
+    for (int b0 = 0; b0 < nblocks; b0 += GS_FINAL_BLOCKS) {
+        const int n = min(GS_FINAL_BLOCKS, nblocks - b0);
+        __syncthreads();  // part is still read by the last round
+#pragma unroll
+        for (int r = 0; r < (GS_FINAL_BLOCKS * GS_NPART + GS_BLOCK - 1) / GS_BLOCK; r++)
+            if (r * GS_BLOCK + t < n * GS_NPART)
+                part[r * GS_BLOCK + t] = partials[(size_t)b0 * GS_NPART + r * GS_BLOCK + t];
+        __syncthreads();
+        if (t < GS_NPART) {
+#pragma unroll 16
+            for (int b = 0; b < n; b++) v += part[b * GS_NPART + t];
+        }
     }
+    if (t < GS_NPART) tot[t] = v;
     __syncthreads();
-    if (threadIdx.x == 0) gs_refine_finish(tot, ubi, n_out, mean_out);
+    if (t == 0) gs_refine_finish(tot, su, ubi, n_out, mean_out);
 }
 
 // One score_and_refine term (src/closest.c:296-316): a peak within tol adds

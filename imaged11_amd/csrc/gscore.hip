@@ -495,7 +495,7 @@ int refine_one_launch(int mode, double* ubi, const double* gv, int ng, double to
         hipLaunchKernelGGL((k_refine_partials<1, false>), dim3(nb), dim3(GS_BLOCK), 0, st, ubi, gv,
                            ng, tolsq, labels, label, partials, nullptr, nullptr);
     GS_LAUNCHED();
-    hipLaunchKernelGGL(k_refine_finalize, dim3(1), dim3(GS_WAVE), 0, st, partials, nb, ubi,
+    hipLaunchKernelGGL(k_refine_finalize, dim3(1), dim3(GS_BLOCK), 0, st, partials, nb, ubi,
                        n_out, mean_out);
     GS_LAUNCHED();
     return GS_OK;
