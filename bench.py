@@ -41,12 +41,6 @@ FLOPS_PER_PAIR = 23      # h = UBI.g: 9 mul + 6 add; 3 sub; sumsq: 3 mul + 2 add
 # pair executed (9 of the 16 k slots carry the split products)
 MFMA_FLOPS_PER_PAIR = 96
 PEAK_F16_MFMA = 2.5e15  # MI355X f16 matrix, dense
-# FP64 VALU instructions per pair of the fused compute_gv + score_and_assign
-# kernel's certified loop, counted in its gfx950 assembly: 70 per grain step
-# of two peaks per lane (22 v_fmac, 16 v_fma, 8 v_mul, 12 v_add, 6
-# v_fract, 2 v_rsq, 4 v_cmp; one Newton step after each v_rsq_f64), plus
-# 2.5 integer VALU per step (the label test of each peak, one LDS address)
-SCAN_VALU_OPS_PER_PAIR = 35.0
 # FP64 flops per list entry of the adjoint pass (hkl-space loss with the
 # Gauss-Newton sums), FMA = 2, counted from its source: forward
 # compute_xlylzl + compute_gv 75, residual and loss 24, dL/dG 18, the
@@ -728,9 +722,9 @@ def aux_scan(threads, with_cpu, K=20000, N=8_000_000, n_iter=20, cpu_peaks=50_00
            "scan_setup_ms": setup,
            "assign_pairs_per_s": K * N / (assign_ms * 1e-3),
            "assign_algorithmic_hbm_gb_s": algo_bytes / (assign_ms * 1e-3) / 1e9,
-           "assign_valu_ops_per_pair": SCAN_VALU_OPS_PER_PAIR,
-           "assign_issued_fp64_ops_frac_of_nonfma_peak":
-               SCAN_VALU_OPS_PER_PAIR * K * N / (assign_ms * 1e-3) / 39.3e12,
+           "assign_mfma_flops_per_pair": MFMA_FLOPS_PER_PAIR,
+           "assign_mfma_frac_of_peak":
+               MFMA_FLOPS_PER_PAIR * K * N / (assign_ms * 1e-3) / PEAK_F16_MFMA,
            "assigned": int((lab >= 0).sum()),
            "own_label_fraction": float(np.mean(lab[own >= 0] == own[own >= 0])),
            "fast_mode_vs_parity_mode": fast_vs_parity,

@@ -18,9 +18,9 @@ Everything after the first selection works on the assigned rows only and
 is vectorised across all tasks at once on the device: the merge is one
 ordered segmented sum per column over (task, key) groups (the reference's
 per-voxel ``np.bincount``, the same sums in the same order), the
-least-squares fits run one task per thread (``gs_pbp_ubi_fit``,
-``gs_pbp_strain_fit``: the task's weighted rows streamed into a QR factor
-by Givens rotations, the factor decomposed by one-sided Jacobi rotations,
+least-squares fits run 16 lanes per task (``gs_pbp_ubi_fit``,
+``gs_pbp_strain_fit``: the task's weighted rows streamed into QR factors by
+Givens rotations, merged, and decomposed by one-sided Jacobi rotations,
 then ``np.linalg.lstsq``'s minimum-norm solution, rank and rcond rule, and
 the reference's cond / det / matrix_rank test of the fitted UBI), and the
 outlier statistics are per-task sums.
