@@ -60,7 +60,8 @@ typedef short gs_short2 __attribute__((ext_vector_type(2)));
 #define GS_SIEVE_ERR_WIDE 0x1p-7
 // The ball (gs_ball_tile) is the faster one from here (1000 x 10^6 at tol 0.1:
 // sieve 207 us, ball 282; at 0.2 a quarter of all quads would pass the sieve),
-// up to where a dead pair's S, 3/4, could come near the tolerance.
+// up to where (tol + sqrt(3) GS_SIEVE_ERR_WIDE)^2, 0.583 at 0.75, would come
+// near a dead pair's S, 3/4.
 #define GS_BALL_TOL_MIN 0.1
 #define GS_BALL_TOL_MAX 0.75
 #define GS_SIEVE_SETS 4    // 32-peak sets per wave (NB)
@@ -269,9 +270,10 @@ __global__ __launch_bounds__(GS_BLOCK) void k_sum_copies(const int* __restrict__
 
 // ---------------------------------------------------------------------------
 // The grains' fragments, packed once per call into the caller's workspace:
-// tile t (grains 32 t .. 32 t + 31; "dead" past K and where u is not finite,
-// as a peak is past the list and where g is not finite: zeros, and 1/2 of h
-// from the p, q slots, which passes no sieve and no ball) has
+// tile t (grains 32 t .. 32 t + 31; "dead" past K and where any of the nine u
+// is not finite, as a peak is past the list and where g is not finite: zeros,
+// and 1/2 of h in all three rows from the p, q slots, which passes no sieve
+// and, as S = 3/4, no ball up to GS_BALL_TOL_MAX) has
 // 3 x 64 x 16 bytes, row-major by UBI row, lane l holding column l & 31 and k
 // slots 8 (l >> 5) .. + 7, then one float per tile, the largest row sum of
 // |u|.  Also clears the counters (so that no separate fill is launched).
@@ -289,10 +291,14 @@ __global__ __launch_bounds__(128) void k_sieve_pack(const double* __restrict__ u
     if (t < 96) {  // one grain row each
         const int row = t / 32, col = t & 31;
         const int g = 32 * tl + col;
-        const double* u = ubis + 9 * (size_t)min(g, K - 1) + 3 * row;
-        double u0 = u[0], u1 = u[1], u2 = u[2];
+        const double* u = ubis + 9 * (size_t)min(g, K - 1);
+        // all three rows: a pair with one row at 1/2 and the others free has
+        // S >= 1/4 only, which the ball counts as certain from tol 1/2 on
+        bool live = g < K;
+#pragma unroll
+        for (int i = 0; i < 9; i++) live = live && gs_finite(u[i]);
+        double u0 = u[3 * row], u1 = u[3 * row + 1], u2 = u[3 * row + 2];
         float a = (float)(fabs(u0) + fabs(u1) + fabs(u2));
-        const bool live = g < K && gs_finite(u0) && gs_finite(u1) && gs_finite(u2);
         if (!live) {
             u0 = u1 = u2 = 0.0;
             a = 0.0f;

@@ -280,6 +280,51 @@ def test_ball_special_values(dev, orc):
             assert np.array_equal(got.cpu().numpy(), orc.score_many(u, g, tol))
 
 
+def nonfinite_inputs():
+    """Three tiles of grains and eight waves of peaks without a huge finite
+    value, so that none of them leaves the matrix cores: in the first tile
+    and its neighbour UBIs with one, two and three rows that are not finite
+    (an entry, a row, entries in both rows), and peaks with one and three
+    components that are not."""
+    ubi, gv = make(96, 1024, 12)
+    n = 0
+    for v in (np.nan, np.inf, -np.inf):
+        for rows in ((0,), (1,), (2,), (0, 1), (1, 2), (0, 2), (0, 1, 2)):
+            ubi[2 * n, rows, n % 3] = v
+            n += 1
+        ubi[50 + n % 7, n % 3] = v  # a whole row
+    for i, v in enumerate((np.nan, np.inf, -np.inf)):
+        gv[40 * i + 3, i] = v
+        gv[40 * i + 300] = v
+    spans = np.abs(np.where(np.isfinite(ubi), ubi, 0.0)).sum(2).max()
+    assert spans * np.abs(gv[np.isfinite(gv)]).max() < 60  # GS_SIEVE_SPAN
+    return ubi, gv
+
+
+@pytest.mark.parametrize("tol", [0.02, 0.1, 0.25, 0.501, 0.55, 0.6, 0.7, 0.709, 0.74])
+def test_nonfinite_values_on_the_matrix_cores(dev, orc, tol):
+    """A pair with a value that is not finite has a NaN drlv2: never counted,
+    whichever rows it leaves finite."""
+    ubi, gv = nonfinite_inputs()
+    for scale in (1.0, 12.0):  # the narrow range and the wide one
+        got = batched.score_sieve(T(ubi * scale, dev), T(gv, dev), tol).cpu().numpy()
+        want = orc.score_many(ubi * scale, gv, tol)
+        assert np.all(want[~np.isfinite(ubi).all((1, 2))] == 0) and want.sum() > 0
+        assert np.array_equal(got, want)
+
+
+@pytest.mark.parametrize("tol", [0.05, 0.25, 0.6, 0.74])
+def test_huge_values_beside_nonfinite_ones(dev, orc, tol):
+    """A huge finite entry in another row of a UBI that is not finite, and in
+    tiles and waves of its own."""
+    ubi, gv = nonfinite_inputs()
+    ubi[0, 1, 1] = 1e300   # beside the NaN of row 0
+    ubi[90, 2, 0] = -1e300
+    gv[900, 1] = 1e300
+    got = batched.score_sieve(T(ubi, dev), T(gv, dev), tol).cpu().numpy()
+    assert np.array_equal(got, orc.score_many(ubi, gv, tol))
+
+
 @pytest.mark.parametrize("tol", [0.125, 0.3, 0.49])
 def test_ball_pairs_on_the_tolerance(dev, orc, tol):
     """Distances that straddle tol by 1e-17 .. 1e-3, along one row, two and

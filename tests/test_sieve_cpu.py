@@ -77,3 +77,21 @@ def test_position_expansion_error_bound(ratio):
     L, A1, T = np.abs(q).sum(1), np.abs(u).sum(1), np.linalg.norm(t, axis=1)
     bound = 1.01 * 2.0 ** -10 * ds / amin * L + 0.5775 * A1 * ds * (T / (amin - T)) ** 2
     assert np.all(np.abs(approx - exact) <= bound + 1e-12)
+
+
+@pytest.mark.parametrize("err", [2.0 ** -11, 2.0 ** -7])
+def test_dead_pairs_lie_beyond_the_ball(err):
+    """A pair held at 1/2 in all three rows has S = 3/4, beyond lo + width at
+    every tolerance the ball takes; held there in one row or two it would
+    be certain from tol 1/2, sqrt(1/2) on, so the three go together."""
+    def units(tol):
+        e = 1.7320508075688774 * err + 1e-9
+        lo = int(max((max(tol - e, 0.0) * 65536.0) ** 2 - 1.0, 0.0))
+        return lo, int(((tol + e) * 65536.0) ** 2 + 2.0)
+
+    for tol in np.linspace(0.1, 0.75, 131):
+        lo, hi = units(tol)
+        assert hi < 3 << 30
+        for dead in (1, 2):  # the live rows at an integer
+            if tol > np.sqrt(dead / 4.0) + 2 * np.sqrt(3.0) * err:
+                assert dead << 30 < lo
