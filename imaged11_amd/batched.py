@@ -39,6 +39,8 @@ from ._lib import SIEVE_TOL_MAX, score_mode  # noqa: E402  (the default score ke
 
 
 MFMA_PAIRS = 16000000  # the least pairs for which the matrix cores pay
+SIEVE_GRAINS_MAX = 1 << 28   # most grains of a score or a selection on them
+ASSIGN_GRAINS_MAX = 1 << 24  # and of an assignment (bits of its queue entries)
 
 
 def mfma_pays(K, N):
@@ -46,8 +48,10 @@ def mfma_pays(K, N):
     peaks.  Its tiles hold 32 grains (4 x 10^6: 20 us against 18 of the row
     sieve, 16 x 10^6: 20 against 31), and its workspace and launches cost the
     host 1.5 to 4 us a call, which is all there is to a small problem (300 x
-    30 000: 18 us against 14, 1000 x 30 000: 17 against 23)."""
-    return K >= 8 and K * N >= MFMA_PAIRS
+    30 000: 18 us against 14, 1000 x 30 000: 17 against 23).  Beyond
+    SIEVE_GRAINS_MAX the kernels without a workspace stay: it takes 97 bytes
+    a grain, more than the UBIs, which alone fill 19 GB there."""
+    return 8 <= K <= SIEVE_GRAINS_MAX and K * N >= MFMA_PAIRS
 
 
 def ball_pays(K, N, tol):
@@ -56,7 +60,8 @@ def ball_pays(K, N, tol):
     against 59 of the all-rows kernel, 1000 x 10^6 290 against 611, 16 x 10^6
     26 against 30; 100 x 160000 took 20 against 18 and 8 x 2 10^6 41 against
     31.  From 0.75 on nearly every pair counts and no caller asks."""
-    return K * N >= 32000000 and K >= 16 and _lib.SIEVE_TOL_MAX < abs(float(tol)) < 0.75
+    return (K * N >= 32000000 and 16 <= K <= SIEVE_GRAINS_MAX
+            and _lib.SIEVE_TOL_MAX < abs(float(tol)) < 0.75)
 
 
 def assign_mfma_pays(K, N, tol):
@@ -65,7 +70,7 @@ def assign_mfma_pays(K, N, tol):
     the FP64 loop (10 x 8e6 with positions: 280 us against 172, 16 x 1e6: 39
     against 41, 777 x 10^5: 90 against 337), and beyond tol 0.12 too many pairs
     pass (500 x 200003: 240 us against 351 at 0.1, 449 against 401 at 0.15)."""
-    return K >= 16 and abs(float(tol)) <= SIEVE_TOL_MAX
+    return 16 <= K <= ASSIGN_GRAINS_MAX and abs(float(tol)) <= SIEVE_TOL_MAX
 
 
 def score_sieve(ubis, gv, tol, out=None):

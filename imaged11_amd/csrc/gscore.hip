@@ -318,6 +318,8 @@ int launch_sieve(const double* ubis, int K, const double* gv, int ng, double tol
     DeviceCtx* ctx;
     GS_CHECK(get_ctx(&ctx));
     if (K < 0 || ng < 0) return set_err(GS_ERR_ARG, "negative size K=%d ng=%d", K, ng);
+    // grains are rounded up to whole tiles in 32 bits
+    if (K > 0x7fffffff - 31) return set_err(GS_ERR_ARG, "the sieve takes at most 2^31 - 32 grains");
     if (K == 0 || ng == 0) return fill_i32(counts, 0, K, st);
     if (!ws || (reinterpret_cast<uintptr_t>(ws) & 15))
         return set_err(GS_ERR_ARG, "the sieve needs a 16-byte aligned workspace");

@@ -136,7 +136,8 @@ int gs_score_many(const double *ubis, int K, const double *gv, int ng, double to
 /* gs_score_many on the matrix cores: the sieve up to |tol| = 0.1, the ball
  * beyond (the reference's counts at any tol).  ws: device memory of at
  * least gs_sieve_workspace_bytes(K) bytes, 16-byte aligned, whose contents
- * need not be kept and may be reused by later work on the stream. */
+ * need not be kept and may be reused by later work on the stream.
+ * K <= 2^31 - 32. */
 long long gs_sieve_workspace_bytes(int K);
 int gs_score_many_ws(const double *ubis, int K, const double *gv, int ng, double tol,
                      int *counts, void *ws, gs_stream_t stream);

@@ -3,6 +3,8 @@ products exact, f32 accumulation that rounds or truncates at every step."""
 import numpy as np
 import pytest
 
+from imaged11_amd import batched
+
 
 def split16(v):
     hi = np.float16(np.float32(v))
@@ -95,3 +97,14 @@ def test_dead_pairs_lie_beyond_the_ball(err):
         for dead in (1, 2):  # the live rows at an integer
             if tol > np.sqrt(dead / 4.0) + 2 * np.sqrt(3.0) * err:
                 assert dead << 30 < lo
+
+
+def test_dispatch_stays_within_the_limits_of_the_kernels():
+    """The queue entries of the assignment hold 24 bits of grain; the score's
+    workspace is larger than the UBIs."""
+    for K, assign, score in ((1 << 24, True, True), ((1 << 24) + 1, False, True),
+                             (1 << 28, False, True), ((1 << 28) + 1, False, False),
+                             ((1 << 31) - 1, False, False), (7, False, False)):
+        assert batched.assign_mfma_pays(K, 10 ** 7, 0.05) == assign
+        assert batched.mfma_pays(K, 10 ** 7) == score
+        assert batched.ball_pays(K, 10 ** 7, 0.3) == score
