@@ -58,12 +58,6 @@ struct gs_tile_info {
     float pad;
 };
 
-// LDS stores of this wave's lanes before, loads after
-__device__ __forceinline__ void gs_wave_sync() {
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-}
-
 __device__ __forceinline__ float gs_uniform(float v) {
     return __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, v)));
 }

@@ -44,7 +44,8 @@
 // finite stand-in.  Larger A: up to GS_SIEVE_SPAN_WIDE the accumulator
 // starts at 1.5 2^27 (its last bit 2^-12 of h) and the fields are shifted
 // left by four first, error GS_SIEVE_ERR_WIDE = 2^-7 by the same count;
-// beyond that every pair takes the reference arithmetic.
+// beyond that, and beyond |u| and |g|, the tile is tested in f32 on the
+// vector ALU (gs_tile32).
 #pragma once
 #include "gs_kernels.h"
 
@@ -126,6 +127,12 @@ __device__ __forceinline__ void gs_grain_frag(double u0, double u1, double u2, c
     b[0] = l[2];
 #pragma unroll
     for (int i = 0; i < 7; i++) b[1 + i] = q ? (_Float16)(float)q[i] : (_Float16)0;
+}
+
+// LDS stores of this wave's lanes before, loads after
+__device__ __forceinline__ void gs_wave_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
 }
 
 __device__ __forceinline__ bool gs_finite(double a) { return fabs(a) < __builtin_inf(); }
@@ -239,6 +246,143 @@ __device__ __forceinline__ int gs_ball_tile(gs_half8 pk, gs_half8 b0, gs_half8 b
     return n;
 }
 
+// ---------------------------------------------------------------------------
+// Tiles outside the f16 ranges, in f32 on the vector ALU: a lane holds one
+// grain of the tile (lane & 31) and goes through the wave's peaks, the lower
+// half of the wave through the even quads and the upper half through the odd
+// ones, with the queue and the entries of gs_sieve_tile.
+// Certification, v = 2^-24 (half a unit in the last place), A = max over rows
+// of |u|_1, times max |g|: u and g are rounded once (2 v A), the three FMAs
+// round a partial sum of at most A + 1 each: h is within 5.1 v A + 3.1 v,
+// below gs_err32 = 2^-21 A + 10^-6, which also covers v_fract_f32 and the
+// rounding of r.  Used while A <= 2^16 (gs_err32 < 0.032) and the factors
+// are far from the ends of f32; beyond that every pair of the grain passes.
+// A grain that is not finite passes nothing; a peak that is not finite is NaN
+// here, which fails every comparison.
+// 14 f32 instructions per pair (ball 21), three 16-byte LDS reads per quad.
+// 1000 grains x 10^6 peaks with cells of 300 to 1200 A: 392 us at tol 0.05,
+// 525 at 0.25; k_score_many_sieve and k_score_many_fast take 449 and 713, and
+// with the reference arithmetic for every pair of the tile it was 1287 and 1413.
+struct gs_grain32 {
+    float u[9];  // zero where the range above does not hold
+    float a;     // A, infinite there
+    bool live;   // all nine finite
+};
+
+__device__ __forceinline__ gs_grain32 gs_load_grain32(const double* __restrict__ u, bool on,
+                                                      float gmax) {
+    gs_grain32 w;
+    double s[3], big = 0.0;
+#pragma unroll
+    for (int i = 0; i < 3; i++) {
+        s[i] = fabs(u[3 * i]) + fabs(u[3 * i + 1]) + fabs(u[3 * i + 2]);
+        big += s[i];
+    }
+    w.live = on && gs_finite(u[0]) && gs_finite(u[1]) && gs_finite(u[2]) && gs_finite(u[3]) &&
+             gs_finite(u[4]) && gs_finite(u[5]) && gs_finite(u[6]) && gs_finite(u[7]) &&
+             gs_finite(u[8]);
+    const double top = fmax(s[0], fmax(s[1], s[2])) * (double)gmax * (1.0 + 0x1p-20);
+    const bool fits = w.live && big < 0x1p100 && gmax < 0x1p100f && top <= 65536.0;
+    w.a = fits ? (float)top : __builtin_inff();
+#pragma unroll
+    for (int i = 0; i < 9; i++) w.u[i] = fits ? (float)u[i] : 0.0f;
+    return w;
+}
+
+// a component of a peak: within the range above or at its end, so that it
+// gives no NaN against a grain of zeros
+__device__ __forceinline__ float gs_clamp32(double v) {
+    return fminf(fmaxf((float)v, -0x1p100f), 0x1p100f);
+}
+
+__device__ __forceinline__ float gs_err32(float a) { return 0x1p-21f * a + 1e-6f; }
+
+// the largest of the fractions of h_i + r
+__device__ __forceinline__ float gs_cube32(const float* u, float x, float y, float z, float r) {
+    const float h0 = __builtin_fmaf(u[2], z, __builtin_fmaf(u[1], y, __builtin_fmaf(u[0], x, r)));
+    const float h1 = __builtin_fmaf(u[5], z, __builtin_fmaf(u[4], y, __builtin_fmaf(u[3], x, r)));
+    const float h2 = __builtin_fmaf(u[8], z, __builtin_fmaf(u[7], y, __builtin_fmaf(u[6], x, r)));
+    return fmaxf(fmaxf(__builtin_amdgcn_fractf(h0), __builtin_amdgcn_fractf(h1)),
+                 __builtin_amdgcn_fractf(h2));
+}
+
+// drlv2 - 3/4, as gs_drlv2_fract
+__device__ __forceinline__ float gs_drlv2_32(const float* u, float x, float y, float z) {
+    const float h0 = __builtin_fmaf(u[2], z, __builtin_fmaf(u[1], y, __builtin_fmaf(u[0], x, 0.5f)));
+    const float h1 = __builtin_fmaf(u[5], z, __builtin_fmaf(u[4], y, __builtin_fmaf(u[3], x, 0.5f)));
+    const float h2 = __builtin_fmaf(u[8], z, __builtin_fmaf(u[7], y, __builtin_fmaf(u[6], x, 0.5f)));
+    const float f0 = __builtin_amdgcn_fractf(h0), f1 = __builtin_amdgcn_fractf(h1),
+                f2 = __builtin_amdgcn_fractf(h2);
+    float t = __builtin_fmaf(f0, f0, -f0);
+    t = __builtin_fmaf(f1, f1, t) - f1;
+    return __builtin_fmaf(f2, f2, t) - f2;
+}
+
+// 32 peaks (x, y, z: theirs, 16-byte aligned) against the tile.  Sieve: a quad
+// is queued unless the fraction of every pair exceeds hi = 2 r (r in lo).
+// Ball: queued if the drlv2 - 3/4 of a pair lies in [lo, hi); returns how many
+// pairs lie below lo in the quads that are not.
+template <bool BALL, class Entry>
+__device__ __forceinline__ int gs_tile32(const float* x, const float* y, const float* z,
+                                         const gs_grain32& w, float lo, float hi, int half,
+                                         unsigned lp, Entry* q, int& qn) {
+    int n = 0;
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        const int pk = 8 * j + 4 * half;
+        bool in;
+        int n4 = 0;
+        if constexpr (BALL) {
+            // s - lo as a bit pattern: negative ones and NaN lie beyond hi - lo
+            unsigned d = 0xffffffffu;
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const float s = gs_drlv2_32(w.u, x[pk + i], y[pk + i], z[pk + i]);
+                n4 += s < lo;
+                d = min(d, __builtin_bit_cast(unsigned, s - lo));
+            }
+            in = d < __builtin_bit_cast(unsigned, hi - lo);
+        } else {
+            float f = gs_cube32(w.u, x[pk], y[pk], z[pk], lo);
+#pragma unroll
+            for (int i = 1; i < 4; i++)
+                f = fminf(f, gs_cube32(w.u, x[pk + i], y[pk + i], z[pk + i], lo));
+            in = f <= hi;
+        }
+        const unsigned long long m = __builtin_amdgcn_ballot_w64(in);
+        if (m) {
+            if (in) {
+                const unsigned pos = __builtin_amdgcn_mbcnt_hi(
+                    (unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u));
+                (q + qn)[pos] = (Entry)(lp + 2 * j);
+                n4 = 0;
+            }
+            qn += __popcll(m);
+        }
+        n += n4;
+    }
+    return n;
+}
+
+// lo and hi of gs_tile32 for the lane's grain at tolerance tol: everything
+// passes beyond the range, nothing where the grain is not finite
+template <bool BALL>
+__device__ __forceinline__ void gs_units32(const gs_grain32& w, double tol, float& lo, float& hi) {
+    const float e = gs_err32(w.a);
+    if constexpr (BALL) {
+        // the roots are off by sqrt(3) e, the sum's own rounding is below 10^-6
+        const float d = 1.7320509f * e, t = (float)tol, a = fmaxf(t - d, 0.0f);
+        lo = fminf(a * a, 4.0f) - 0.750002f;
+        hi = fminf((t + d) * (t + d), 4.0f) - 0.749998f;
+        if (!w.live) lo = hi = -2.0f;  // below every drlv2 - 3/4
+    } else {
+        const float r = (float)tol + e;
+        lo = r < 0.49f ? r : 0.0f;
+        hi = r < 0.49f ? 2.0f * r + 1e-6f : 2.0f;
+        if (!w.live) hi = -1.0f;
+    }
+}
+
 __device__ __forceinline__ gs_float16 gs_splat16(float v) {
     return (gs_float16){v, v, v, v, v, v, v, v, v, v, v, v, v, v, v, v};
 }
@@ -339,7 +483,9 @@ __global__ __launch_bounds__(GS_BLOCK, 4) void k_score_mfma(
     constexpr int NB = GS_SIEVE_SETS;
     static_assert(8 * NB <= 32, "a queue entry holds 5 bits of quad");
     static_assert(32 * GS_SIEVE_SPLIT <= 2048, "and 11 bits of grain");
+    static_assert(GS_SIEVE_SPLIT <= GS_WAVE, "a lane looks at one tile's span");
     __shared__ __align__(16) gs_half8 lpk[NW][NB][GS_WAVE];
+    __shared__ __align__(16) float lf[NW][3][32 * NB];  // the peaks for gs_tile32
     __shared__ int lcnt[32 * GS_SIEVE_SPLIT];
     __shared__ unsigned short lq[NW][GS_WAVE + 256];
     const int tile = gs_xcd_remap(blockIdx.x, gridDim.x);
@@ -355,6 +501,7 @@ __global__ __launch_bounds__(GS_BLOCK, 4) void k_score_mfma(
     // this wave's peaks: k0 .. k0 + 32 NB - 1
     const long long k0 = (long long)chunk * (NW * NB * 32) + wave * (NB * 32);
     float gmax = 0.0f;
+    const float sl = span[min(t0 + lane, t1 - 1)];  // lane l: of tile t0 + l
     for (int s = 0; s < NB; s++) {
         long long k = k0 + 32 * s + (lane & 31);
         bool live = k < ng;
@@ -369,6 +516,16 @@ __global__ __launch_bounds__(GS_BLOCK, 4) void k_score_mfma(
     for (int o = 1; o < 32; o <<= 1) gmax = fmaxf(gmax, __shfl_xor(gmax, o, GS_WAVE));
     gmax = __builtin_bit_cast(
         float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, gmax * (1.0f + 0x1p-20f))));
+    // the peaks in f32, if a tile of the split is tested so
+    if (__ballot(!(sl < GS_SIEVE_UMAX && gmax < GS_SIEVE_GMAX && sl * gmax <= GS_SIEVE_SPAN_WIDE)))
+        for (int p = lane; p < 32 * NB; p += GS_WAVE) {
+            const long long k = min(k0 + p, (long long)ng - 1);
+            const double x = gv[3 * k], y = gv[3 * k + 1], z = gv[3 * k + 2];
+            const bool live = k0 + p < ng && gs_finite(x) && gs_finite(y) && gs_finite(z);
+            lf[wave][0][p] = live ? gs_clamp32(x) : __builtin_nanf("");
+            lf[wave][1][p] = gs_clamp32(y);
+            lf[wave][2][p] = gs_clamp32(z);
+        }
     const double tol = sqrt(tolsq) * (1.0 + 1e-15) + 1e-12;
     int r16, thr, r16w, thrw;
     gs_sieve_units(tol + GS_SIEVE_ERR, r16, thr);
@@ -450,13 +607,16 @@ __global__ __launch_bounds__(GS_BLOCK, 4) void k_score_mfma(
                 drain();
             }
         } else {
-            for (int g = 32 * t; g < min(K, 32 * t + 32); g++) {
-                const gs_ubi u = gs_load_ubi(ubis + 9 * (size_t)g);
-                for (int s = 0; s < NB * 32; s += GS_WAVE) {
-                    const long long k = k0 + s + lane;
-                    if (k < ng && gs_drlv2(u, gv[3 * k], gv[3 * k + 1], gv[3 * k + 2]) < tolsq)
-                        hit(g - g0, k);
-                }
+            const int g = min(32 * t + (lane & 31), K - 1);
+            const gs_grain32 w =
+                gs_load_grain32(ubis + 9 * (size_t)g, 32 * t + (lane & 31) < K, gmax);
+            float l32, h32;
+            gs_units32<BALL>(w, tol, l32, h32);
+#pragma unroll 1
+            for (int s = 0; s < NB; s++) {
+                n += gs_tile32<BALL>(lf[wave][0] + 32 * s, lf[wave][1] + 32 * s,
+                                     lf[wave][2] + 32 * s, w, l32, h32, half, lp + 8 * s, q, qn);
+                drain();
             }
         }
         if (BALL && n) atomicAdd(&lcnt[32 * (t - t0) + (lane & 31)], n);

@@ -325,6 +325,56 @@ def test_huge_values_beside_nonfinite_ones(dev, orc, tol):
     assert np.array_equal(got, orc.score_many(ubi, gv, tol))
 
 
+# tiles past the f16 ranges, tested in f32: spans from just beyond them to
+# where f32 says nothing, factors up to the ends of f32 and past them
+@pytest.mark.parametrize("cell,gmax", [((700.0, 1100.0), 1.6), ((3.0, 9.0), 40.0),
+                                       ((0.3, 0.9), 90.0), ((9e3, 2.5e4), 1.6),
+                                       ((3e4, 3e5), 1.6), ((1e28, 3e28), 1e-27),
+                                       ((1e33, 3e33), 1e-32), ((1e-32, 3e-32), 1e33),
+                                       ((1e-44, 3e-44), 1e45), ((1e40, 3e40), 1e-39)])
+@pytest.mark.parametrize("K,N", [(33, 129), (64, 1000), (95, 2049)])
+def test_tiles_in_f32(dev, orc, cell, gmax, K, N):
+    ubi, gv = make(K, N, K, cell=cell, gmax=gmax)
+    for tol in (0.0, 0.02, 0.1, 0.15, 0.45, 0.74):
+        got = batched.score_sieve(T(ubi, dev), T(gv, dev), tol)
+        want = orc.score_many(ubi, gv, tol)
+        assert tol < 0.1 or want.sum() > 0
+        assert np.array_equal(got.cpu().numpy(), want)
+
+
+@pytest.mark.parametrize("tol", [0.02, 0.1, 0.25, 0.6, 0.74])
+def test_nonfinite_values_in_f32(dev, orc, tol):
+    """The same values in tiles that are tested in f32, beside grains in
+    range and grains whose every pair is settled."""
+    ubi, gv = nonfinite_inputs()
+    ubi[:32] *= 300.0  # past the f16 ranges
+    ubi[32:64:5] *= 1e5  # and those of f32
+    ubi[61, 1, 1], gv[900, 1] = 1e300, -1e300
+    got = batched.score_sieve(T(ubi, dev), T(gv, dev), tol).cpu().numpy()
+    want = orc.score_many(ubi, gv, tol)
+    assert want[:32].sum() > 0 and want[64:].sum() > 0
+    assert np.array_equal(got, want)
+
+
+@pytest.mark.parametrize("cell,gmax", [((700.0, 1100.0), 1.6), ((0.3, 0.9), 90.0),
+                                       ((3e4, 3e5), 1.6)])
+def test_selected_lists_in_f32(dev, cell, gmax):
+    from imaged11_amd import indexing
+    K, N, tol = 700, 30001, 0.05
+    ubi, gv = make(K, N, 2, cell=cell, gmax=gmax)
+    u, g = T(ubi, dev), T(gv, dev)
+    assert batched.mfma_pays(K, N)
+    idx, off = indexing.select_lists(u, g, tol * tol)
+    n = batched.score_many(u, g, tol, exact=True)
+    assert np.array_equal(np.diff(off.cpu().numpy()), n.cpu().numpy())
+    for k in range(0, K, 97):
+        h = gv @ ubi[k].T
+        d = ((h - np.rint(h)) ** 2).sum(1)
+        got = idx[off[k]:off[k + 1]].cpu().numpy()
+        scale = 1e-15 * np.abs(ubi[k]).sum() * np.abs(gv).max()  # of h in float64
+        assert np.abs(d - tol * tol).min() < scale or np.array_equal(got, np.nonzero(d < tol * tol)[0])
+
+
 @pytest.mark.parametrize("tol", [0.125, 0.3, 0.49])
 def test_ball_pairs_on_the_tolerance(dev, orc, tol):
     """Distances that straddle tol by 1e-17 .. 1e-3, along one row, two and

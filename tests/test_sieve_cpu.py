@@ -81,6 +81,45 @@ def test_position_expansion_error_bound(ratio):
     assert np.all(np.abs(approx - exact) <= bound + 1e-12)
 
 
+def fma32(a, b, c):
+    """f32 FMA: the product of two f32 is exact in f64 (the sum's rounding there
+    is 2^-29 of the rounding to f32)."""
+    return (a.astype(np.float64) * b.astype(np.float64) + c).astype(np.float32)
+
+
+@pytest.mark.parametrize("span", [1e-3, 1.0, 60.0, 1000.0, 16384.0, 65536.0])
+def test_f32_tile_error_bound(span):
+    """h + r of gs_cube32 within 2^-21 A + 10^-6, and drlv2 of gs_drlv2_32
+    within the bounds gs_units32 draws around it."""
+    rng = np.random.default_rng(3)
+    n, worst = 200000, 0.0
+    u = rng.uniform(-1, 1, (n, 3, 3))
+    g = rng.uniform(-1, 1, (n, 3))
+    g[::3] = np.sign(u[::3, 0]) * np.abs(g[::3]).max(1)[:, None]  # the largest sums
+    u *= span / (np.abs(u).sum(2).max(1) * np.abs(g).max(1))[:, None, None]
+    A = np.abs(u).sum(2).max(1) * np.abs(g).max(1)
+    err = 2.0 ** -21 * A + 1e-6
+    u32, g32 = u.astype(np.float32), g.astype(np.float32)
+    f, d2 = [], []
+    for row in range(3):
+        exact = (u[:, row].astype(np.longdouble) * g.astype(np.longdouble)).sum(1)
+        for start in (0.0501, 0.5):
+            h = np.full(n, start, np.float32)
+            for j in range(3):
+                h = fma32(u32[:, row, j], g32[:, j], h.astype(np.float64))
+            worst = max(worst, float((np.abs(h - (exact + np.float32(start))) / err).max()))
+        f.append(h - np.floor(h))
+        d2.append((exact - np.rint(exact)) ** 2)
+    assert 0.05 < worst < 0.99
+    t = fma32(f[0], f[0], -f[0].astype(np.float64))
+    for k in (1, 2):
+        t = fma32(f[k], f[k], t.astype(np.float64)) - f[k]
+    root = np.sqrt(sum(d2).astype(float))
+    d = 1.7320509 * err
+    assert np.all(t >= np.maximum(root - d, 0) ** 2 - 0.750002)
+    assert np.all(t <= (root + d) ** 2 - 0.749998)
+
+
 @pytest.mark.parametrize("err", [2.0 ** -11, 2.0 ** -7])
 def test_dead_pairs_lie_beyond_the_ball(err):
     """A pair held at 1/2 in all three rows has S = 3/4, beyond lo + width at
