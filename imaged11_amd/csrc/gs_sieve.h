@@ -428,33 +428,42 @@ __global__ __launch_bounds__(128) void k_sieve_pack(const double* __restrict__ u
                                                     gs_half8* __restrict__ frag,
                                                     float* __restrict__ span,
                                                     int* __restrict__ counts, int copies) {
-    __shared__ float lspan[96];
+    __shared__ float lspan[128];  // largest row sums
+    __shared__ unsigned long long lfin[2];  // bit per lane: the thread's row is finite
     const int tl = blockIdx.x, t = threadIdx.x;
+    const int row = t / 32, col = t & 31;
+    double u0 = 0.0, u1 = 0.0, u2 = 0.0;
+    float sp = 0.0f;
+    if (t < 96) {  // one grain row each
+        const double* u = ubis + 9 * (size_t)min(32 * tl + col, K - 1) + 3 * row;
+        u0 = u[0];
+        u1 = u[1];
+        u2 = u[2];
+    }
     if (32 * tl + (t & 31) < K)
         for (int c = t / 32; c < copies; c += 4) counts[(size_t)c * K + 32 * tl + (t & 31)] = 0;
-    if (t < 96) {  // one grain row each
-        const int row = t / 32, col = t & 31;
-        const int g = 32 * tl + col;
-        const double* u = ubis + 9 * (size_t)min(g, K - 1);
+    const unsigned long long fin = __ballot(gs_finite(u0) && gs_finite(u1) && gs_finite(u2));
+    if ((t & (GS_WAVE - 1)) == 0) lfin[t / GS_WAVE] = fin;
+    __syncthreads();
+    if (t < 96) {
         // all three rows: a pair with one row at 1/2 and the others free has
         // S >= 1/4 only, which the ball counts as certain from tol 1/2 on
-        bool live = g < K;
-#pragma unroll
-        for (int i = 0; i < 9; i++) live = live && gs_finite(u[i]);
-        double u0 = u[3 * row], u1 = u[3 * row + 1], u2 = u[3 * row + 2];
+        const bool live = 32 * tl + col < K &&
+                          (lfin[0] >> col & lfin[0] >> (32 + col) & lfin[1] >> col & 1);
         float a = (float)(fabs(u0) + fabs(u1) + fabs(u2));
         if (!live) {
             u0 = u1 = u2 = 0.0;
             a = 0.0f;
         }
         const double q[7] = {live ? 1.0 : 0.0, live ? 0.0 : 32768.0, 0.0, 0.0, 0.0, 0.0, 0.0};
-        lspan[t] = a * (1.0f + 0x1p-20f);
+        sp = a * (1.0f + 0x1p-20f);
         gs_half8* f = frag + (3 * (size_t)tl + row) * GS_WAVE;
         gs_half8 lo, hi;
         gs_grain_frag(u0, u1, u2, q, lo, hi);
         f[col] = lo;
         f[col + 32] = hi;
     }
+    lspan[t] = sp;
     __syncthreads();
     if (t == 0) {
         float a = lspan[0];
