@@ -492,7 +492,7 @@ __global__ __launch_bounds__(GS_BLOCK, 4) void k_score_mfma(
     constexpr int NB = GS_SIEVE_SETS;
     static_assert(8 * NB <= 32, "a queue entry holds 5 bits of quad");
     static_assert(32 * GS_SIEVE_SPLIT <= 2048, "and 11 bits of grain");
-    static_assert(GS_SIEVE_SPLIT <= GS_WAVE, "a lane looks at one tile's span");
+    static_assert(GS_SIEVE_SPLIT <= 64, "a mask holds the tiles left to f32");
     __shared__ __align__(16) gs_half8 lpk[NW][NB][GS_WAVE];
     __shared__ __align__(16) float lf[NW][3][32 * NB];  // the peaks for gs_tile32
     __shared__ int lcnt[32 * GS_SIEVE_SPLIT];
@@ -510,7 +510,6 @@ __global__ __launch_bounds__(GS_BLOCK, 4) void k_score_mfma(
     // this wave's peaks: k0 .. k0 + 32 NB - 1
     const long long k0 = (long long)chunk * (NW * NB * 32) + wave * (NB * 32);
     float gmax = 0.0f;
-    const float sl = span[min(t0 + lane, t1 - 1)];  // lane l: of tile t0 + l
     for (int s = 0; s < NB; s++) {
         long long k = k0 + 32 * s + (lane & 31);
         bool live = k < ng;
@@ -525,16 +524,6 @@ __global__ __launch_bounds__(GS_BLOCK, 4) void k_score_mfma(
     for (int o = 1; o < 32; o <<= 1) gmax = fmaxf(gmax, __shfl_xor(gmax, o, GS_WAVE));
     gmax = __builtin_bit_cast(
         float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, gmax * (1.0f + 0x1p-20f))));
-    // the peaks in f32, if a tile of the split is tested so
-    if (__ballot(!(sl < GS_SIEVE_UMAX && gmax < GS_SIEVE_GMAX && sl * gmax <= GS_SIEVE_SPAN_WIDE)))
-        for (int p = lane; p < 32 * NB; p += GS_WAVE) {
-            const long long k = min(k0 + p, (long long)ng - 1);
-            const double x = gv[3 * k], y = gv[3 * k + 1], z = gv[3 * k + 2];
-            const bool live = k0 + p < ng && gs_finite(x) && gs_finite(y) && gs_finite(z);
-            lf[wave][0][p] = live ? gs_clamp32(x) : __builtin_nanf("");
-            lf[wave][1][p] = gs_clamp32(y);
-            lf[wave][2][p] = gs_clamp32(z);
-        }
     const double tol = sqrt(tolsq) * (1.0 + 1e-15) + 1e-12;
     int r16, thr, r16w, thrw;
     gs_sieve_units(tol + GS_SIEVE_ERR, r16, thr);
@@ -547,6 +536,7 @@ __global__ __launch_bounds__(GS_BLOCK, 4) void k_score_mfma(
     }
     unsigned short* q = lq[wave];
     int qn = 0;
+    unsigned long long left = 0;  // the split's tiles that the loop over them leaves out
     const auto hit = [&](int gl, long long k) {
         if constexpr (SELECT) {
             const int g = g0 + gl;
@@ -616,19 +606,37 @@ __global__ __launch_bounds__(GS_BLOCK, 4) void k_score_mfma(
                 drain();
             }
         } else {
-            const int g = min(32 * t + (lane & 31), K - 1);
+            left |= 1ull << (t - t0);
+        }
+        if (BALL && n) atomicAdd(&lcnt[32 * (t - t0) + (lane & 31)], n);
+    }
+    if (left) {  // the tiles outside the f16 ranges, here so that the loop above has the registers
+        for (int p = lane; p < 32 * NB; p += GS_WAVE) {
+            const long long k = min(k0 + p, (long long)ng - 1);
+            const double x = gv[3 * k], y = gv[3 * k + 1], z = gv[3 * k + 2];
+            const bool live = k0 + p < ng && gs_finite(x) && gs_finite(y) && gs_finite(z);
+            lf[wave][0][p] = live ? gs_clamp32(x) : __builtin_nanf("");
+            lf[wave][1][p] = gs_clamp32(y);
+            lf[wave][2][p] = gs_clamp32(z);
+        }
+        gs_wave_sync();
+        for (; left; left &= left - 1) {
+            const int tl = __builtin_ctzll(left);
+            const int g = g0 + 32 * tl + (lane & 31);
             const gs_grain32 w =
-                gs_load_grain32(ubis + 9 * (size_t)g, 32 * t + (lane & 31) < K, gmax);
+                gs_load_grain32(ubis + 9 * (size_t)min(g, K - 1), g < K, gmax);
             float l32, h32;
             gs_units32<BALL>(w, tol, l32, h32);
+            const unsigned lp = ((32 * tl + (lane & 31)) << 5) | half;
+            int n = 0;
 #pragma unroll 1
             for (int s = 0; s < NB; s++) {
                 n += gs_tile32<BALL>(lf[wave][0] + 32 * s, lf[wave][1] + 32 * s,
                                      lf[wave][2] + 32 * s, w, l32, h32, half, lp + 8 * s, q, qn);
                 drain();
             }
+            if (BALL && n) atomicAdd(&lcnt[32 * tl + (lane & 31)], n);
         }
-        if (BALL && n) atomicAdd(&lcnt[32 * (t - t0) + (lane & 31)], n);
     }
     __builtin_amdgcn_wave_barrier();
     if (lane < qn) settle(q[lane]);
