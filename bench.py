@@ -905,7 +905,7 @@ def main():
     pairs = args.grains * args.peaks
     value = pairs * args.steps / (total_ms * 1e-3)
     if (batched.score_mode(args.tol) == _lib.SCORE_SIEVE and
-            batched.mfma_pays(args.grains, args.peaks)):
+            batched.score_mfma_pays(args.grains, args.peaks, args.tol)):
         kernel, bound, peak = "k_score_mfma", "mfma", PEAK_F16_MFMA
         achieved = MFMA_FLOPS_PER_PAIR * pairs / (score_ms * 1e-3)
         frac_is = ("f16 matrix flops executed over the dense f16 peak; the kernel's vector "

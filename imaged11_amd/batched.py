@@ -38,29 +38,54 @@ def _ready():
 from ._lib import SIEVE_TOL_MAX, score_mode  # noqa: E402  (the default score kernel)
 
 
-MFMA_PAIRS = 16000000  # the least pairs for which the matrix cores pay
+MFMA_PAIRS = 16000000  # below, nothing takes the matrix cores but the assignment
 SIEVE_GRAINS_MAX = 1 << 28   # most grains of a score or a selection on them
 ASSIGN_GRAINS_MAX = 1 << 24  # and of an assignment (bits of its queue entries)
 
 
 def mfma_pays(K, N):
-    """Whether the matrix-core sieve is the faster one for K grains x N
-    peaks.  Its tiles hold 32 grains (4 x 10^6: 20 us against 18 of the row
-    sieve, 16 x 10^6: 20 against 31), and its workspace and launches cost the
-    host 1.5 to 4 us a call, which is all there is to a small problem (300 x
-    30 000: 18 us against 14, 1000 x 30 000: 17 against 23).  Beyond
-    SIEVE_GRAINS_MAX the kernels without a workspace stay: it takes 97 bytes
-    a grain, more than the UBIs, which alone fill 19 GB there."""
+    """Whether the matrix-core sieve is the faster one for the lists of K
+    grains x N peaks (indexing.select_lists: 1.1 to 2 times the row sieve from
+    here on, K = 8 to 3000).  Beyond SIEVE_GRAINS_MAX the kernels without a
+    workspace stay: it takes 97 bytes a grain, more than the UBIs, which alone
+    fill 19 GB there."""
     return 8 <= K <= SIEVE_GRAINS_MAX and K * N >= MFMA_PAIRS
+
+
+def score_mfma_pays(K, N, tol):
+    """Whether the counts of K grains x N peaks are faster on the matrix cores
+    (score_sieve) than by the row sieve.  Each line lies where the ratio of
+    the times (row sieve over matrix cores; peaks of the grains and random
+    ones, tol 0.02 / 0.05 / 0.1) passes 1; the row sieve has its grains in
+    splits of 8, the matrix cores in tiles of 32:
+    * up to one tile: K = 16 1.10 / 1.24 / 1.25 at 16 x 10^6 pairs, 31 1.04 /
+      1.15 / 1.17; K = 12 0.8 at any size;
+    * two or three tiles, the last one partly empty, where the splits come out
+      even: K = 40 0.8 at 64 x 10^6 and 1.1 at 96 x 10^6, 48 0.9 and 72 1.0
+      there;
+    * others up to 256, with a launch for the sum of their counters: 44 1.1 at
+      24 x 10^6, 64 0.99 / 1.05 / 1.13; 160 0.93 / 1.14 / 1.17 at 32 x 10^6,
+      100 0.89 / 1.0 / 0.99 there and 0.94 / 1.04 / 1.01 at 48 x 10^6;
+    * beyond 256: 1000 0.85 / 0.84 / 0.94 at 16 x 10^6, 1.06 / 1.11 / 1.18 at
+      18 x 10^6, and 1.9 at 128 x 10^6."""
+    pairs, wide = K * N, abs(float(tol)) >= 0.04
+    if K <= 32:
+        return K >= 16 and pairs >= MFMA_PAIRS
+    if K > 256:
+        return K <= SIEVE_GRAINS_MAX and pairs >= 18000000
+    if K < 96 and K % 8 == 0 and K % 32:
+        return pairs >= 96000000
+    return pairs >= (24000000 if K <= 64 else 32000000 if wide else 48000000)
 
 
 def ball_pays(K, N, tol):
     """Whether the matrix cores pay beyond the sieves' tolerances, where the
-    ball counts the pairs (gs_ball_tile): 257 x 300007 at tol 0.25 40 us
-    against 59 of the all-rows kernel, 1000 x 10^6 290 against 611, 16 x 10^6
-    26 against 30; 100 x 160000 took 20 against 18 and 8 x 2 10^6 41 against
-    31.  From 0.75 on nearly every pair counts and no caller asks."""
-    return (K * N >= 32000000 and 16 <= K <= SIEVE_GRAINS_MAX
+    ball counts the pairs (gs_ball_tile): 257 x 300007 at tol 0.25 41 us
+    against 59 of the all-rows kernel, 1000 x 10^6 290 against 611.  At the
+    line 1.3 (16 grains) to 0.96 (48); 40 grains, five even splits of the
+    other kernel, 0.89 there and 1.2 at 96 x 10^6; 8 x 2 10^6 41 against 31.
+    From tol 0.75 on nearly every pair counts and no caller asks."""
+    return (16 <= K <= SIEVE_GRAINS_MAX and K * N >= (96000000 if K == 40 else 32000000)
             and _lib.SIEVE_TOL_MAX < abs(float(tol)) < 0.75)
 
 
@@ -95,7 +120,7 @@ def score_many(ubis, gv, tol, peaks_per_lane=0, out=None, exact=False, mode=None
     ubis (K,3,3) float64, gv (N,3) float64 -> int32 (K,).  exact=True uses
     the reference's arithmetic for every pair; by default the certified
     kernel score_mode(tol) picks runs; every mode returns the reference's
-    counts.  mfma_pays and ball_pays say when the matrix cores take the
+    counts.  score_mfma_pays and ball_pays say when the matrix cores take the
     call instead (a tile height peaks_per_lane asks for the kernels on the
     vector ALU, and so does mode=SCORE_CERTIFIED)."""
     lib = _ready()
@@ -112,7 +137,7 @@ def score_many(ubis, gv, tol, peaks_per_lane=0, out=None, exact=False, mode=None
         ball = False
     # (the pairs first: a small problem's time is this host code)
     if K * N >= MFMA_PAIRS and not peaks_per_lane and (
-            mode == _lib.SCORE_SIEVE and mfma_pays(K, N) or ball and ball_pays(K, N, tol)):
+            mode == _lib.SCORE_SIEVE and score_mfma_pays(K, N, tol) or ball and ball_pays(K, N, tol)):
         return score_sieve(ubis, gv, tol, out)
     _lib.check(lib.gs_score_many(dptr(ubis), K, dptr(gv), N, float(tol), dptr(out),
                                  int(peaks_per_lane), mode, stream_ptr()), "score_many")

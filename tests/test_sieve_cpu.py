@@ -146,4 +146,22 @@ def test_dispatch_stays_within_the_limits_of_the_kernels():
                              ((1 << 31) - 1, False, False), (7, False, False)):
         assert batched.assign_mfma_pays(K, 10 ** 7, 0.05) == assign
         assert batched.mfma_pays(K, 10 ** 7) == score
+        assert batched.score_mfma_pays(K, 10 ** 7, 0.05) == score
         assert batched.ball_pays(K, 10 ** 7, 0.3) == score
+
+
+@pytest.mark.parametrize("K,pairs,narrow,wide", [
+    (1, 10 ** 9, False, False), (15, 10 ** 8, False, False), (16, 16 * 10 ** 6, True, True),
+    (16, 15999984, False, False), (32, 16 * 10 ** 6, True, True), (33, 23 * 10 ** 6, False, False),
+    (33, 24 * 10 ** 6, True, True), (40, 64 * 10 ** 6, False, False), (40, 96 * 10 ** 6, True, True),
+    (64, 24 * 10 ** 6, True, True), (72, 95 * 10 ** 6, False, False),
+    (88, 96 * 10 ** 6, True, True), (96, 32 * 10 ** 6, False, True),
+    (100, 48 * 10 ** 6, True, True), (256, 31 * 10 ** 6, False, False),
+    (256, 48 * 10 ** 6, True, True), (257, 17 * 10 ** 6, False, False),
+    (1000, 18 * 10 ** 6, True, True), (12000, 15 * 10 ** 6, False, False)])
+def test_the_score_takes_the_matrix_cores_where_they_were_measured_faster(K, pairs, narrow, wide):
+    """Both sides of every line of the rule."""
+    N = -(-pairs // K)
+    for sign in (1, -1):
+        assert batched.score_mfma_pays(K, N, sign * 0.02) == narrow
+        assert batched.score_mfma_pays(K, N, sign * 0.05) == wide
