@@ -295,6 +295,8 @@ __device__ __forceinline__ float gs_clamp32(double v) {
     return fminf(fmaxf((float)v, -0x1p100f), 0x1p100f);
 }
 
+#define GS_ALL32 2.0f  // hi of a grain whose every pair passes
+
 __device__ __forceinline__ float gs_err32(float a) { return 0x1p-21f * a + 1e-6f; }
 
 // the largest of the fractions of h_i + r
@@ -316,6 +318,20 @@ __device__ __forceinline__ float gs_drlv2_32(const float* u, float x, float y, f
     float t = __builtin_fmaf(f0, f0, -f0);
     t = __builtin_fmaf(f1, f1, t) - f1;
     return __builtin_fmaf(f2, f2, t) - f2;
+}
+
+// the entries of the lanes with `in` to the end of the wave's queue
+template <class Entry>
+__device__ __forceinline__ void gs_push(bool in, Entry e, Entry* q, int& qn) {
+    const unsigned long long m = __builtin_amdgcn_ballot_w64(in);
+    if (m) {
+        if (in) {
+            const unsigned pos = __builtin_amdgcn_mbcnt_hi(
+                (unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u));
+            (q + qn)[pos] = e;
+        }
+        qn += __popcll(m);
+    }
 }
 
 // 32 peaks (x, y, z: theirs, 16-byte aligned) against the tile.  Sieve: a quad
@@ -349,26 +365,19 @@ __device__ __forceinline__ int gs_tile32(const float* x, const float* y, const f
                 f = fminf(f, gs_cube32(w.u, x[pk + i], y[pk + i], z[pk + i], lo));
             in = f <= hi;
         }
-        const unsigned long long m = __builtin_amdgcn_ballot_w64(in);
-        if (m) {
-            if (in) {
-                const unsigned pos = __builtin_amdgcn_mbcnt_hi(
-                    (unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u));
-                (q + qn)[pos] = (Entry)(lp + 2 * j);
-                n4 = 0;
-            }
-            qn += __popcll(m);
-        }
+        if (in) n4 = 0;
+        gs_push(in, (Entry)(lp + 2 * j), q, qn);
         n += n4;
     }
     return n;
 }
 
-// lo and hi of gs_tile32 for the lane's grain at tolerance tol: everything
-// passes beyond the range, nothing where the grain is not finite
+// lo and hi of gs_tile32 for the lane's grain at tolerance tol and error e of
+// a row: everything passes beyond the range (e infinite), nothing where the
+// grain is not finite
 template <bool BALL>
-__device__ __forceinline__ void gs_units32(const gs_grain32& w, double tol, float& lo, float& hi) {
-    const float e = gs_err32(w.a);
+__device__ __forceinline__ void gs_units32(const gs_grain32& w, double tol, float e, float& lo,
+                                           float& hi) {
     if constexpr (BALL) {
         // the roots are off by sqrt(3) e, the sum's own rounding is below 10^-6
         const float d = 1.7320509f * e, t = (float)tol, a = fmaxf(t - d, 0.0f);
@@ -378,7 +387,7 @@ __device__ __forceinline__ void gs_units32(const gs_grain32& w, double tol, floa
     } else {
         const float r = (float)tol + e;
         lo = r < 0.49f ? r : 0.0f;
-        hi = r < 0.49f ? 2.0f * r + 1e-6f : 2.0f;
+        hi = r < 0.49f ? 2.0f * r + 1e-6f : GS_ALL32;
         if (!w.live) hi = -1.0f;
     }
 }
@@ -626,7 +635,7 @@ __global__ __launch_bounds__(GS_BLOCK, 4) void k_score_mfma(
             const gs_grain32 w =
                 gs_load_grain32(ubis + 9 * (size_t)min(g, K - 1), g < K, gmax);
             float l32, h32;
-            gs_units32<BALL>(w, tol, l32, h32);
+            gs_units32<BALL>(w, tol, gs_err32(w.a), l32, h32);
             const unsigned lp = ((32 * tl + (lane & 31)) << 5) | half;
             int n = 0;
 #pragma unroll 1

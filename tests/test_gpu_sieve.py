@@ -169,6 +169,73 @@ def test_scan_over_positions_and_cells(dev, orc, dist, t, cell):
     assert want.sum() > 300
 
 
+# lengths, cells and wavelengths towards the ends of f32 and past them; one
+# detector distance of positions beyond |a| / 2
+@pytest.mark.parametrize("dist,t,cell,wvln", [(8000.0, 500.0, (3.0, 9.0), 0.2),
+                                              (8000.0, 500.0, (3e2, 9e3), 0.2),
+                                              (8000.0, 500.0, (3e4, 9e4), 0.2),
+                                              (8e-9, 5e-10, (3.0, 9.0), 0.2),
+                                              (8e-14, 5e-15, (3.0, 9.0), 0.2),
+                                              (8e12, 5e11, (3.0, 9.0), 0.2),
+                                              (8e17, 5e16, (3.0, 9.0), 0.2),
+                                              (8000.0, 500.0, (3e-15, 9e-15), 2e-16),
+                                              (8000.0, 500.0, (3e20, 9e20), 2e19),
+                                              (8000.0, 6000.0, (3.0, 9.0), 0.2)])
+@pytest.mark.parametrize("K,N", [(33, 130), (100, 3001), (40, 140001)])
+def test_scan_tiles_in_f32(dev, orc, dist, t, cell, wvln, K, N):
+    ubi, trans, xl, so, co, w, rng = scan_inputs(K, N, K, dist=dist, t=t, cell=cell, wvln=wvln)
+    l0 = rng.integers(-2, K + 2, N).astype(np.int32)
+    want = check_scan(dev, orc, ubi, trans, xl, so, co, w, 0.1, np.full(N, 2.0), l0)
+    assert want.sum() > 0
+
+
+@pytest.mark.parametrize("dist,t", [(150000.0, 200.0), (8000.0, 500.0)])
+def test_scan_of_grains_far_off(dev, orc, dist, t):
+    """One, then a third of the grains far from the others (by 0.4 and by 3
+    detector distances): tiles of both kinds in one wave."""
+    K, N = 170, 4000
+    ubi, trans, xl, so, co, w, rng = scan_inputs(K, N, 5, dist=dist, t=t)
+    for far in (np.array([77]), np.arange(0, K, 3)):
+        for by in (0.4, 3.0):
+            tr = trans.copy()
+            tr[far, 1] = by * dist
+            check_scan(dev, orc, ubi, tr, xl, so, co, w, 0.1, np.full(N, 2.0),
+                       np.full(N, -1, np.int32))
+
+
+@pytest.mark.parametrize("dist", [150000.0, 8000.0])
+def test_scan_nonfinite_values_on_both_routes(dev, orc, dist):
+    """Values that are not finite without a huge one beside them."""
+    K, N = 96, 2000
+    ubi, trans, xl, so, co, w, rng = scan_inputs(K, N, 9, dist=dist, t=500.0)
+    for i, v in enumerate((np.nan, np.inf, -np.inf)):
+        xl[200 * i + 7, i] = v
+        so[200 * i + 60] = co[200 * i + 77] = v
+        ubi[7 * i, i] = v
+        ubi[7 * i + 1, i, 0] = v
+        trans[7 * i + 2, i] = v
+        trans[7 * i + 3] = v
+    want = check_scan(dev, orc, ubi, trans, xl, so, co, w, 0.1, np.full(N, 2.0),
+                      rng.integers(-2, K + 2, N).astype(np.int32))
+    assert want.sum() > 0
+
+
+@pytest.mark.parametrize("scale", [1.0, 300.0, 1e6])
+def test_assignment_nonfinite_values(dev, orc, scale):
+    """The same for g-vectors given: on the matrix cores, in f32, settled."""
+    ubi, gv = nonfinite_inputs()
+    ubi, K, N = ubi * scale, len(ubi), len(gv)
+    rng = np.random.default_rng(1)
+    d0, l0 = rng.uniform(0, 0.02, N), rng.integers(-2, K + 2, N).astype(np.int32)
+    d, lab = d0.copy(), l0.copy()
+    want = orc.assign_many(ubi, np.arange(K), gv, 0.1, d, lab)
+    dd, ll = T(d0, dev), T(l0, dev, torch.int32)
+    got = batched.assign_many(T(ubi, dev), T(gv, dev), 0.1, dd, ll)
+    assert want.sum() > 0 and np.array_equal(got.cpu().numpy(), want)
+    assert np.array_equal(ll.cpu().numpy(), lab)
+    assert np.array_equal(dd.cpu().numpy().view(np.int64), d.view(np.int64))
+
+
 def test_scan_from_other_states(dev, orc):
     """Labels of the grains and others, current drlv2 anywhere in reach,
     repeated grains, peaks and grains with special values, a peak at the

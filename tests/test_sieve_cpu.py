@@ -120,6 +120,40 @@ def test_f32_tile_error_bound(span):
     assert np.all(t <= (root + d) ** 2 - 0.749998)
 
 
+@pytest.mark.parametrize("ratio", [1e-3, 0.05, 0.3, 0.5])
+@pytest.mark.parametrize("cell", [3.0, 300.0, 12000.0])
+def test_f32_position_error_bound(ratio, cell):
+    """u.G of the assignment's f32 tiles, |t| up to half of |a|, with the
+    inverse square root off by its 2 v either way: within 2^-19 A1 ds."""
+    rng = np.random.default_rng(4)
+    n, ds, amin = 100000, 5.0, 8000.0
+    a = rng.normal(size=(n, 3))
+    a *= (amin * rng.uniform(1.0, 3.0, n) / np.linalg.norm(a, axis=1))[:, None]
+    t = rng.normal(size=(n, 3))
+    t *= (ratio * amin * rng.uniform(0.0, 1.0, n) / np.linalg.norm(t, axis=1))[:, None]
+    t[::3] = a[::3] * (ratio * amin / np.linalg.norm(a[::3], axis=1))[:, None]  # towards it
+    c = rng.normal(size=(n, 3))
+    c *= ds / np.linalg.norm(c, axis=1)[:, None]
+    u = rng.uniform(-cell, cell, (n, 3))
+    e = (a - t).astype(np.longdouble)
+    G = ds * e / np.sqrt((e * e).sum(1))[:, None] - c
+    exact = (u * G).sum(1)
+    f = np.float32
+    e32 = a.astype(f) - t.astype(f)
+    n2 = e32[:, 0] * e32[:, 0]
+    for j in (1, 2):
+        n2 = fma32(e32[:, j], e32[:, j], n2.astype(np.float64))
+    for off in (-1.0, 0.0, 1.0):
+        rsq = (1.0 / np.sqrt(n2.astype(np.float64)) * (1.0 + off * 2.0 ** -23)).astype(f)
+        inv = f(ds) * rsq
+        h = np.full(n, f(0.0501))
+        for j in range(3):
+            g = fma32(e32[:, j], inv, -c[:, j].astype(f).astype(np.float64))
+            h = fma32(u[:, j].astype(f), g, h.astype(np.float64))
+        err = np.abs(h - f(0.0501) - exact) / (2.0 ** -19 * np.abs(u).sum(1) * ds + 1e-6)
+        assert 0.02 < err.max() < 0.99
+
+
 @pytest.mark.parametrize("err", [2.0 ** -11, 2.0 ** -7])
 def test_dead_pairs_lie_beyond_the_ball(err):
     """A pair held at 1/2 in all three rows has S = 3/4, beyond lo + width at
