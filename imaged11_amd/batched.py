@@ -92,10 +92,13 @@ def ball_pays(K, N, tol):
 def assign_mfma_pays(K, N, tol):
     """Whether the assignment behind the matrix-core sieve is the faster one
     for K grains x N peaks.  A peak's fragments cost as much as ~10 grains of
-    the FP64 loop (10 x 8e6 with positions: 280 us against 172, 16 x 1e6: 39
-    against 41, 777 x 10^5: 90 against 337), and beyond tol 0.12 too many pairs
-    pass (500 x 200003: 240 us against 351 at 0.1, 449 against 401 at 0.15)."""
-    return 16 <= K <= ASSIGN_GRAINS_MAX and abs(float(tol)) <= SIEVE_TOL_MAX
+    the FP64 loop (10 x 8e6 with positions: 280 us against 172, 16 x 1e6: 66
+    against 61, 24 x 1e6: 66 against 75, 777 x 10^5: 90 against 337), up to 19
+    grains the more so the more peaks there are (16 x 4 10^6: 204 us against
+    155), and beyond tol 0.12 too many pairs pass (500 x 200003: 240 us against
+    351 at 0.1, 449 against 401 at 0.15)."""
+    return (16 <= K <= ASSIGN_GRAINS_MAX and abs(float(tol)) <= SIEVE_TOL_MAX
+            and (K >= 20 or N <= 300000))
 
 
 def score_sieve(ubis, gv, tol, out=None):

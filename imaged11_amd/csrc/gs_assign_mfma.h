@@ -32,7 +32,7 @@
 // from the ends of f32; otherwise every pair of the grain passes.  Measured,
 // 2000 grains x 10^6 peaks 8 mm from the detector, positions to 500 um: 1761 us
 // against 2973 of k_gv_assign_many and 3498 with its FP64 loop for such tiles
-// here; g-vectors given, cells of 300 to 1200 A: 763 against 2191 and 2259.
+// here; g-vectors given, cells of 300 to 1200 A: 813 against 2149 and 2259.
 //
 // Order.  The update rule is sequential in the grains of one peak: a pair is
 // accepted if its drlv2 is below tol^2 and the peak's current drlv2, so the
@@ -145,9 +145,12 @@ __global__ __launch_bounds__(128) void k_assign_pack(const double* __restrict__ 
     }
 }
 
-// NB 32 peaks per wave, all K grains.  gvx: the g-vectors, or with GEOM the
+// NB 32 peaks per wave, all K grains.  FEW: at most 64 of them, counted in LDS:
+// with many peaks of each their atomics went one after the other (16 grains x
+// 4 10^6 peaks of theirs 577 us, 204 this way; as a branch at run time it cost
+// 777 grains x 10^5 with positions a tenth).  gvx: the g-vectors, or with GEOM the
 // lab positions (so, co, gp then given as for k_gv_assign_many).
-template <bool GEOM, int NB>
+template <bool GEOM, int NB, bool FEW>
 __global__ __launch_bounds__(GS_BLOCK, 3) void k_assign_mfma(
     const double* __restrict__ gvx, const double* __restrict__ so_in,
     const double* __restrict__ co_in, int ng, gs_goniometer gp, const double* __restrict__ ubis,
@@ -164,6 +167,7 @@ __global__ __launch_bounds__(GS_BLOCK, 3) void k_assign_mfma(
     __shared__ double ld[NW][NP];                           // current drlv2
     __shared__ int lg[NW][NP];                              // last accepted grain, or -1
     __shared__ unsigned lclaim[NW][NP];
+    __shared__ int lcnt[FEW ? NW : 1][GS_WAVE];  // the wave's counts
     __shared__ unsigned lq1[NW][GS_WAVE + 256];  // grain << 5 | quad
     __shared__ unsigned lq2[NW][2 * GS_WAVE];    // grain << 7 | peak
     const int lane = threadIdx.x & (GS_WAVE - 1);
@@ -173,6 +177,7 @@ __global__ __launch_bounds__(GS_BLOCK, 3) void k_assign_mfma(
     if (k0 >= ng) return;  // no barrier of the block below
     const double* mat = gp.mat;
     const double ds = 1. / gp.wvln;
+    if (FEW) lcnt[wave][lane] = 0;
     unsigned* q1 = lq1[wave];
     unsigned* q2 = lq2[wave];
 
@@ -273,7 +278,10 @@ __global__ __launch_bounds__(GS_BLOCK, 3) void k_assign_mfma(
         if (se < ld[wave][pk]) {
             ld[wave][pk] = se;
             lg[wave][pk] = g;
-            atomicAdd(&counts[g], 1);
+            if constexpr (FEW)
+                atomicAdd(&lcnt[wave][g], 1);
+            else
+                atomicAdd(&counts[g], 1);
         }
     };
     int n1 = 0, n2 = 0;  // fills of the queues, wave-uniform
@@ -381,7 +389,6 @@ __global__ __launch_bounds__(GS_BLOCK, 3) void k_assign_mfma(
     const float ds32 = GEOM ? (float)ds : 0.0f, cz32 = GEOM ? (float)(ds * mat[2]) : 0.0f;
     const bool range32 = GEOM && n2min > 0x1p-80 && n2max < 0x1p100 && fabs(ds) > 0x1p-60 &&
                          fabs(ds) < 0x1p60;
-    bool have32 = false;  // lf holds g
     int radii = 0;  // lane l: the radius of tile (t & ~63) + l
     for (int t = 0; t < tiles; t++) {
         const gs_half8 b0 = m0, b1 = m1, b2 = m2;
@@ -424,18 +431,15 @@ __global__ __launch_bounds__(GS_BLOCK, 3) void k_assign_mfma(
                 t2 = (float)tr[2];
                 gs_units32<false>(w, tol, fits ? 4.0f * gs_err32(w.a) : __builtin_inff(), lo, hi);
             } else {
-                if (!have32) {
-                    for (int p = lane; p < NP; p += GS_WAVE) {
-                        const long long k = min(k0 + p, (long long)ng - 1);
-                        const double x = gvx[3 * k], y = gvx[3 * k + 1], z = gvx[3 * k + 2];
-                        const bool live = gs_finite(x) && gs_finite(y) && gs_finite(z);
-                        lf[wave][0][p] = live ? gs_clamp32(x) : __builtin_nanf("");
-                        lf[wave][1][p] = gs_clamp32(y);
-                        lf[wave][2][p] = gs_clamp32(z);
-                    }
-                    have32 = true;
-                    gs_wave_sync();
-                }
+                for (int p = lane; p < NP; p += GS_WAVE) {
+                const long long k = min(k0 + p, (long long)ng - 1);
+                const double x = gvx[3 * k], y = gvx[3 * k + 1], z = gvx[3 * k + 2];
+                const bool live = gs_finite(x) && gs_finite(y) && gs_finite(z);
+                lf[wave][0][p] = live ? gs_clamp32(x) : __builtin_nanf("");
+                lf[wave][1][p] = gs_clamp32(y);
+                lf[wave][GEOM ? 0 : 2][p] = gs_clamp32(z);
+            }
+                gs_wave_sync();
                 w = gs_load_grain32(ubis + 9 * (size_t)g, on, gmax);
                 gs_units32<false>(w, tol, gs_err32(w.a), lo, hi);
             }
@@ -470,6 +474,8 @@ __global__ __launch_bounds__(GS_BLOCK, 3) void k_assign_mfma(
     }
     flush();
     gs_wave_sync();
+    if constexpr (FEW)
+        if (lane < K && lcnt[wave][lane]) atomicAdd(&counts[lane], lcnt[wave][lane]);
     for (int pk = lane; pk < NP; pk += GS_WAVE) {
         const long long k = k0 + pk;
         if (k < ng) {

@@ -422,14 +422,14 @@ int launch_assign_many(const double* ubis, const int* glabels, int K, const doub
 // matrix-core sieve: the pack launch, which also clears counts, and the
 // pairs.  32, 64 or 128 peaks per wave: the largest that still gives every
 // SIMD two waves.
-template <bool GEOM, int NB>
+template <bool GEOM, int NB, bool FEW>
 int launch_assign_nb(const double* gvx, const double* so, const double* co, int ng,
                      const gs_goniometer& gp, const double* ubis, const double* trans, int K,
                      double tolsq, const gs_half8* frag, const gs_tile_info* info,
                      const int* yexp, double* drlv2, int* labels, int* priv, int copies,
                      hipStream_t st) {
     const int nb = blocks_for(ng, 32 * NB * (GS_BLOCK / GS_WAVE));
-    hipLaunchKernelGGL((k_assign_mfma<GEOM, NB>), dim3(nb), dim3(GS_BLOCK), 0, st, gvx, so, co, ng,
+    hipLaunchKernelGGL((k_assign_mfma<GEOM, NB, FEW>), dim3(nb), dim3(GS_BLOCK), 0, st, gvx, so, co, ng,
                        gp, ubis, trans, K, tolsq, frag, info, yexp, drlv2, labels, priv, copies);
     GS_LAUNCHED();
     return GS_OK;
@@ -457,9 +457,11 @@ int launch_assign_sieve(const double* gvx, const double* so, const double* co, i
                        info, yexp, priv, copies);
     GS_LAUNCHED();
     const long long waves = 8LL * ctx->cus;
-    const auto pairs = ng >= 128 * waves  ? launch_assign_nb<GEOM, 4>
-                       : ng >= 64 * waves ? launch_assign_nb<GEOM, 2>
-                                          : launch_assign_nb<GEOM, 1>;
+    const bool few = K <= GS_WAVE;
+    const auto pairs =
+        ng >= 128 * waves  ? (few ? launch_assign_nb<GEOM, 4, true> : launch_assign_nb<GEOM, 4, false>)
+        : ng >= 64 * waves ? (few ? launch_assign_nb<GEOM, 2, true> : launch_assign_nb<GEOM, 2, false>)
+                           : (few ? launch_assign_nb<GEOM, 1, true> : launch_assign_nb<GEOM, 1, false>);
     GS_CHECK(pairs(gvx, so, co, ng, gp, ubis, trans, K, tol * tol, frag, info, yexp, drlv2, labels,
                    priv, copies, st));
     hipLaunchKernelGGL(k_sum_copies, dim3(blocks_for(K, GS_BLOCK)), dim3(GS_BLOCK), 0, st, priv,

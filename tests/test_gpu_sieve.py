@@ -272,6 +272,21 @@ def test_assignment_of_gvectors(dev, orc, K, N, tol):
         assert np.array_equal(dd.cpu().numpy().view(np.int64), d.view(np.int64))
 
 
+@pytest.mark.parametrize("K", [19, 20, 63, 64, 65])
+@pytest.mark.parametrize("N", [300000, 300001, 131072, 5000])
+def test_assignment_of_few_grains(dev, K, N):
+    """Counts in LDS up to 64 grains, and the sizes that leave them to the
+    FP64 loop, against the reference arithmetic."""
+    ubi, gv = make(K, N, K, own=0.8)
+    u, g = T(ubi, dev), T(gv, dev)
+    d = [torch.full((N,), 2.0, dtype=torch.float64, device=dev) for _ in range(2)]
+    lab = [torch.full((N,), -1, dtype=torch.int32, device=dev) for _ in range(2)]
+    n = [batched.assign_many(u, g, 0.1, d[i], lab[i], exact=i == 1) for i in range(2)]
+    assert n[1].sum().item() > N / 4
+    for a, b in (n, d, lab):
+        assert torch.equal(a, b)
+
+
 @pytest.mark.parametrize("cell,gmax", [((20.0, 60.0), 1.6), ((300.0, 900.0), 1.6),
                                        ((0.05, 0.2), 40.0)])
 def test_assignment_over_the_ranges_of_the_accumulator(dev, orc, cell, gmax):

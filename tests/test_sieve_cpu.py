@@ -184,6 +184,12 @@ def test_dispatch_stays_within_the_limits_of_the_kernels():
         assert batched.ball_pays(K, 10 ** 7, 0.3) == score
 
 
+def test_few_grains_with_many_peaks_stay_with_the_vector_kernel():
+    for K, N, pays in ((15, 100, False), (16, 300000, True), (19, 300001, False), (20, 10 ** 7, True)):
+        assert batched.assign_mfma_pays(K, N, 0.05) == pays
+        assert not batched.assign_mfma_pays(K, N, 0.11)
+
+
 @pytest.mark.parametrize("K,pairs,narrow,wide", [
     (1, 10 ** 9, False, False), (15, 10 ** 8, False, False), (16, 16 * 10 ** 6, True, True),
     (16, 15999984, False, False), (32, 16 * 10 ** 6, True, True), (33, 23 * 10 ** 6, False, False),
