@@ -12,16 +12,21 @@
 //     p = (ds/|a|) (nx nx, ny ny, nz nz, nx ny, nx nz, ny nz)
 //     q = (ux tx - u.t, uy ty - u.t, uz tz - u.t, ux ty + uy tx,
 //          ux tz + uz tx, uy tz + uz ty)
-// in single f16 numbers, p 2^(16 - y) and q 2^y with 2^y max|t| in [8, 16).
+// in single f16 numbers, p 2^(16 - y) and q 2^y, 2^y between 32 and 64 ds/|a| of
+// a middling peak: p is then below 8192 in the waves whose peaks lie no nearer
+// than a quarter of that, and q below 32768 for every grain that the radius lets
+// through where they lie no farther than 2.5 times.  (From the largest |t| one
+// grain far off made p too large for all: 777 x 10^5 121 us, 200 with one such
+// grain in f32 and 441 in FP64; 121 this way.)
 // Added to the sieve's error (L = max over rows of sum |q|, T = max |t|, A1 =
 // max over rows of |u|_1, in the tile; amin = min |a| over the wave's peaks):
 //   rounding of p and q: 1.01 2^-10 (ds/amin) L;
 //   the remainder of the expansion: for x(s) = a - s t, |d2/ds2 x/|x|| =
 //   |t_perp| sqrt(4 t_par^2 + t_perp^2)/|x|^2 <= 1.1548 |t|^2/|x|^2, so it is
 //   below 0.5775 A1 ds T^2/(amin - T)^2.
-// Terms that f16 flushes (p, q below 2^-14) move h by < 1e-4 while p <= 8192,
-// within the sieve's margin.  The expansion is used while T <= amin/2 and the
-// radius stays below GS_ASSIGN_RMAX; otherwise (grains far from the centre of a
+// Terms that f16 may flush (p, q below 2^-14) move h by 2^-30 (sum |q| + sum p) <
+// 2^-30 (32768 + 2 8192) = 4.6e-5, within the sieve's margin.  The expansion is
+// used while p and sum |q| keep these limits, T <= amin/2 and the radius stays below GS_ASSIGN_RMAX; otherwise (grains far from the centre of a
 // near detector) the tile is tested in f32 on the vector ALU, as in gs_tile32,
 // with G itself from a, t and c.  Its error there, v = 2^-24, while |t| <= |a|/2
 // (so |a| + |t| <= 3 |a - t|): a - t is within 4 v |a - t|, the square of its
@@ -60,6 +65,7 @@
 
 #define GS_ASSIGN_RMAX 0.2f
 #define GS_ASSIGN_PMAX 8192.0f
+#define GS_ASSIGN_QMAX 32768.0f
 
 struct gs_tile_info {
     float span;  // largest row sum of |u|
@@ -73,9 +79,13 @@ __device__ __forceinline__ float gs_uniform(float v) {
 }
 
 // Fragments and tile_info of every tile, the exponent y, the counters cleared.
+// xl (GEOM): the ng peaks, ds = 1/wavelength; y is every block's own, from the
+// median |xl| of the same 128 of them.
 template <bool GEOM>
 __global__ __launch_bounds__(128) void k_assign_pack(const double* __restrict__ ubis,
                                                      const double* __restrict__ trans, int K,
+                                                     const double* __restrict__ xl, int ng,
+                                                     double ds,
                                                      gs_half8* __restrict__ frag,
                                                      gs_tile_info* __restrict__ info,
                                                      int* __restrict__ yexp,
@@ -85,18 +95,24 @@ __global__ __launch_bounds__(128) void k_assign_pack(const double* __restrict__ 
     if (32 * tl + (t & 31) < K)
         for (int c = t / 32; c < copies; c += 4) priv[(size_t)c * K + 32 * tl + (t & 31)] = 0;
     int y = 0;
-    if constexpr (GEOM) {  // 2^y from the largest |t| component of all grains
-        float m = 0.0f;
-        for (long long i = t; i < 3LL * K; i += 128) {
-            const float v = (float)fabs(trans[i]);
-            m = v < __builtin_inff() ? fmaxf(m, v) : m;
-        }
-        lt[t] = m;
+    if constexpr (GEOM) {
+        const double* x = xl + 3 * ((long long)t * ng / 128);
+        const double n2 = x[0] * x[0] + x[1] * x[1] + x[2] * x[2];
+        const float len = n2 > 0.0 ? (float)sqrt(n2) : __builtin_inff();  // NaN: not one either
+        lt[t] = len;
+        if (t == 0) lspan[0] = __builtin_inff();
         __syncthreads();
-        for (int i = 0; i < 128; i++) m = fmaxf(m, lt[i]);
+        int rank = 0, n = 0;
+        for (int i = 0; i < 128; i++) {
+            rank += lt[i] < len || (lt[i] == len && i < t);
+            n += lt[i] < __builtin_inff();
+        }
+        if (rank == n / 2) lspan[0] = len;
+        __syncthreads();
+        const float r = 64.0f * fabsf((float)ds) / lspan[0];
         int e = 0;
-        if (m > 0.0f) (void)frexpf(m, &e);
-        y = m > 0.0f ? max(-60, min(60, 4 - e)) : 0;
+        if (r > 0.0f && r < __builtin_inff()) (void)frexpf(r, &e);
+        y = max(-60, min(60, e - 1));
         if (tl == 0 && t == 0) *yexp = y;
         __syncthreads();
     }
@@ -236,6 +252,7 @@ __global__ __launch_bounds__(GS_BLOCK, 3) void k_assign_mfma(
     const float amin = gs_uniform((float)sqrt(n2min) * (1.0f - 0x1p-20f));
     const float dsa = GEOM ? gs_uniform((float)fabs(ds)) / amin * (1.0f + 0x1p-20f) : 0.0f;
     const float pmax = GEOM ? ldexpf(dsa, 16 - *yexp) : 0.0f;
+    const float lmax = GEOM ? ldexpf(GS_ASSIGN_QMAX, -*yexp) : 0.0f;  // of sum |q|, unscaled
     const float tol = (float)(sqrt(tolsq) + 1e-9);
     gs_wave_sync();
 
@@ -382,7 +399,8 @@ __global__ __launch_bounds__(GS_BLOCK, 3) void k_assign_mfma(
         }
         const bool fits = w.span < GS_SIEVE_UMAX && gmax < GS_SIEVE_GMAX &&
                           sp <= GS_SIEVE_SPAN_WIDE && r < GS_ASSIGN_RMAX &&
-                          (!GEOM || (pmax <= GS_ASSIGN_PMAX && amin > 0.0f && 2.0f * w.tmax <= amin));
+                          (!GEOM || (pmax <= GS_ASSIGN_PMAX && w.lin <= lmax && amin > 0.0f &&
+                                     2.0f * w.tmax <= amin));
         return fits ? (((int)(r * 65536.0f) + 66) & ~63) | (wide ? GS_WIDE : 0) : 0;
     };
     // f32: everything that does not depend on the grain
@@ -432,13 +450,13 @@ __global__ __launch_bounds__(GS_BLOCK, 3) void k_assign_mfma(
                 gs_units32<false>(w, tol, fits ? 4.0f * gs_err32(w.a) : __builtin_inff(), lo, hi);
             } else {
                 for (int p = lane; p < NP; p += GS_WAVE) {
-                const long long k = min(k0 + p, (long long)ng - 1);
-                const double x = gvx[3 * k], y = gvx[3 * k + 1], z = gvx[3 * k + 2];
-                const bool live = gs_finite(x) && gs_finite(y) && gs_finite(z);
-                lf[wave][0][p] = live ? gs_clamp32(x) : __builtin_nanf("");
-                lf[wave][1][p] = gs_clamp32(y);
-                lf[wave][GEOM ? 0 : 2][p] = gs_clamp32(z);
-            }
+                    const long long k = min(k0 + p, (long long)ng - 1);
+                    const double x = gvx[3 * k], y = gvx[3 * k + 1], z = gvx[3 * k + 2];
+                    const bool live = gs_finite(x) && gs_finite(y) && gs_finite(z);
+                    lf[wave][0][p] = live ? gs_clamp32(x) : __builtin_nanf("");
+                    lf[wave][1][p] = gs_clamp32(y);
+                    lf[wave][GEOM ? 0 : 2][p] = gs_clamp32(z);
+                }
                 gs_wave_sync();
                 w = gs_load_grain32(ubis + 9 * (size_t)g, on, gmax);
                 gs_units32<false>(w, tol, gs_err32(w.a), lo, hi);

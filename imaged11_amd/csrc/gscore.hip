@@ -453,8 +453,8 @@ int launch_assign_sieve(const double* gvx, const double* so, const double* co, i
     int* yexp = reinterpret_cast<int*>(info + tiles);
     int* priv = yexp + 4;
     const int copies = gs_copies(K);
-    hipLaunchKernelGGL(k_assign_pack<GEOM>, dim3(tiles), dim3(128), 0, st, ubis, trans, K, frag,
-                       info, yexp, priv, copies);
+    hipLaunchKernelGGL(k_assign_pack<GEOM>, dim3(tiles), dim3(128), 0, st, ubis, trans, K, gvx, ng,
+                       GEOM ? 1.0 / gp.wvln : 0.0, frag, info, yexp, priv, copies);
     GS_LAUNCHED();
     const long long waves = 8LL * ctx->cus;
     const bool few = K <= GS_WAVE;

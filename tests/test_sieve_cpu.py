@@ -81,6 +81,42 @@ def test_position_expansion_error_bound(ratio):
     assert np.all(np.abs(approx - exact) <= bound + 1e-12)
 
 
+@pytest.mark.parametrize("window", [8.0, 32.0, 64.0, 160.0])
+@pytest.mark.parametrize("ratio", [1e-4, 0.01, 0.06])
+def test_position_expansion_over_the_exponents(window, ratio):
+    """The same with 2^y anywhere between 8 and 160 ds/|a|, numbers below the
+    normal f16 range flushed to zero: p within 8192, sum |q| within 32768
+    wherever the radius stays below 0.2, and the flushed terms within their
+    2^-30 (32768 + 2 8192)."""
+    rng = np.random.default_rng(5)
+    n, ds, amin = 20000, 5.0, 150000.0
+    a = rng.normal(size=(n, 3))
+    a *= (amin * rng.uniform(1.0, 1.3, n) / np.linalg.norm(a, axis=1))[:, None]
+    t = rng.normal(size=(n, 3)) * 10.0 ** rng.uniform(-9, 0, (n, 3))
+    t *= (ratio * amin * rng.uniform(0.0, 1.0, n) / np.linalg.norm(t, axis=1))[:, None]
+    u = rng.uniform(-9, 9, (n, 3)) * 10.0 ** rng.uniform(-6, 0, (n, 3))
+    y = int(np.floor(np.log2(window * ds / amin)))
+    if 2.0 ** y < 8 * ds / amin:
+        y += 1
+    r = np.linalg.norm(a, axis=1)
+    nn = a / r[:, None]
+    i, j = np.array([0, 1, 2, 0, 0, 1]), np.array([0, 1, 2, 1, 2, 2])
+    p = (ds / r)[:, None] * nn[:, i] * nn[:, j]
+    q = u[:, i] * t[:, j] + u[:, j] * t[:, i]
+    q[:, :3] = u * t - (u * t).sum(1)[:, None]
+    L = np.abs(q).sum(1)
+    sieved = 1.01 * 2.0 ** -10 * ds / amin * L < 0.2
+    f = lambda v: np.float16(np.float32(v)).astype(float)
+    p16, q16 = f(p * 2.0 ** (16 - y)), f(q * 2.0 ** y)
+    assert np.abs(p16).max() <= 8192 and (L * 2.0 ** y)[sieved].max() <= 32768
+    near = (p16 * q16).sum(1) / 65536.0
+    flush = lambda v: np.where(np.abs(v) < 2.0 ** -14, 0.0, v)
+    gone = np.abs((flush(p16) * flush(q16)).sum(1) / 65536.0 - near)
+    assert gone[sieved].max() <= 2.0 ** -30 * (32768 + 2 * 8192)
+    err = np.abs(near - (p * q).sum(1)) - 1.01 * 2.0 ** -10 * ds / amin * L
+    assert err[sieved].max() <= 2.0 ** -30 * (32768 + 2 * 8192)
+
+
 def fma32(a, b, c):
     """f32 FMA: the product of two f32 is exact in f64 (the sum's rounding there
     is 2^-29 of the rounding to f32)."""
