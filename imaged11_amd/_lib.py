@@ -133,6 +133,8 @@ SIGNATURES = {
                                _vp, _i, _vp, _vp]),
     "gs_pbp_ubi_fit": (_i, [_vp, _vp, _vp, _vp, _dp, _i, _vp, _vp, _vp, _vp, _vp, _vp]),
     "gs_pbp_strain_fit": (_i, [_vp, _vp, _vp, _i, _vp, _vp]),
+    "gs_pbp_ubi_fit_lanes": (_i, [_vp, _vp, _vp, _vp, _dp, _i, _i, _vp, _vp, _vp, _vp, _vp, _vp]),
+    "gs_pbp_strain_fit_lanes": (_i, [_vp, _vp, _vp, _i, _i, _vp, _vp]),
     "gs_pbp_rows_dot": (_i, [_vp, _vp, ctypes.c_longlong, _vp, _d, _vp, _vp, _vp, _vp]),
     "gs_segment_sum": (_i, [_vp, _i, _vp, _i, _vp, _vp]),
     "gs_segment_max": (_i, [_vp, _i, _vp, _i, _vp, _vp]),

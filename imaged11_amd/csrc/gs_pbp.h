@@ -163,7 +163,7 @@ __global__ __launch_bounds__(GS_BLOCK) void k_pbp_merge_sums(const long long* __
 }
 
 // ---------------------------------------------------------------------------
-// The per-task least-squares fits of refine_map, GS_FIT_LANES lanes per task,
+// The per-task least-squares fits of refine_map, LANES lanes per task,
 // solved as np.linalg.lstsq solves them: the minimum-norm solution with
 // the singular values of the weighted design matrix below rcond * the
 // largest taken as zero, rcond = eps * max(rows, columns).  Each task's
@@ -171,11 +171,16 @@ __global__ __launch_bounds__(GS_BLOCK) void k_pbp_merge_sums(const long long* __
 // rotations, the right-hand sides carried along as extra columns), and R,
 // which has the design matrix's singular values, is decomposed by one-sided
 // Jacobi rotations.  Nothing squares the condition number.  A lane takes
-// every GS_FIT_LANES-th row of its task; the lanes' triangular factors are
-// merged the same way, by a tree, and the first lane solves.  With a thread
-// per task the 3100 tasks of a 61 x 61 map were 49 waves, each a serial chain
-// of ~150 rows of square roots and divisions: 496 us for the UBI fit and 935
-// for the strain fit; with 16 lanes 71 and 183 us (refine_map 7.47 -> 6.32 ms).
+// every LANES-th row of its task; the lanes' triangular factors are merged the
+// same way, by a tree, and the first lane solves.
+// One lane is a serial chain over the rows (square roots and divisions), which
+// 16 lanes shorten while they leave SIMDs idle; but all of them merge, and the
+// solver has one in 16 of its lanes at work, so that many tasks or few rows
+// want one.  UBI fit / strain fit in us with 1, 4 and 16 lanes:
+//   3100 tasks x 400 rows  289 86 65 / 499 188 182;  x 20  29 25 49 / 69 - 148
+//   10 000 x 60   53 34 63 / 115 79 226;  20 000 x 150  142 73 134 / 225 293 365
+//   200 000 x 20  116 203 655 / 295 602 2178
+// point_by_point.fit_lanes draws the lines.
 
 // Rotate one row x[0..NC+NR) into the upper-triangular [R | C].
 template <int NC, int NR>
@@ -217,14 +222,13 @@ __device__ __forceinline__ void gs_qr_add_rows(double (&R)[NC][NC + NR],
     }
 }
 
-// [R | C] of the GS_FIT_LANES lanes of a task (aligned, all of them here)
+// [R | C] of the LANES lanes of a task (aligned, all of them here)
 // into the first lane's: at each step a lane rotates in the rows of the lane
 // `o` away, whose factor then holds the same number of the task's rows.
-#define GS_FIT_LANES 16
-template <int NC, int NR>
+template <int NC, int NR, int LANES>
 __device__ __forceinline__ void gs_qr_merge(double (&R)[NC][NC + NR]) {
 #pragma unroll 1
-    for (int o = 1; o < GS_FIT_LANES; o <<= 1) {
+    for (int o = 1; o < LANES; o <<= 1) {
         double other[NC][NC + NR];
 #pragma unroll
         for (int i = 0; i < NC; i++)
@@ -396,13 +400,14 @@ struct gs_mat9 {
 // ubifit (NaN when not fitted), lstsq's rank, worth = rank 3, cond < 1e14,
 // det > 0 and matrix_rank 3; ubi_out = ubifit when worth, else ubi_in; and
 // ub0 = U.B0 of ubifit when worth (NaN otherwise).
+template <int LANES>
 __global__ __launch_bounds__(64) void k_pbp_ubi_fit(
     const double* __restrict__ design, const long long* __restrict__ off,
     const int* __restrict__ fit, const double* __restrict__ ubi_in, gs_mat9 B0, int T,
     double* __restrict__ ubifit, int* __restrict__ rank_out, int* __restrict__ worth_out,
     double* __restrict__ ubi_out, double* __restrict__ ub0) {
-    const int t = (blockIdx.x * 64 + threadIdx.x) / GS_FIT_LANES;
-    const int sl = threadIdx.x & (GS_FIT_LANES - 1);
+    const int t = blockIdx.x * (64 / LANES) + threadIdx.x / LANES;
+    const int sl = threadIdx.x & (LANES - 1);
     const bool on = t < T && fit[t];
     double R[3][6];
 #pragma unroll
@@ -410,8 +415,8 @@ __global__ __launch_bounds__(64) void k_pbp_ubi_fit(
 #pragma unroll
         for (int j = 0; j < 6; j++) R[i][j] = 0.0;
     const long long r0 = on ? off[t] : 0, r1 = on ? off[t + 1] : 0;
-    gs_qr_add_rows<3, 3, 4>(R, design, r0 + sl, r1, GS_FIT_LANES);
-    gs_qr_merge<3, 3>(R);  // every lane of the wave
+    gs_qr_add_rows<3, 3, LANES == 1 ? 8 : 4>(R, design, r0 + sl, r1, LANES);
+    gs_qr_merge<3, 3, LANES>(R);  // every lane of the wave
     if (t >= T || sl) return;
     double u[9], uo[9], b0[9];
     for (int i = 0; i < 9; i++) {
@@ -456,12 +461,13 @@ __global__ __launch_bounds__(64) void k_pbp_ubi_fit(
 // The strain fit of refine_map (:1652-1656) for every task with
 // worth[t] != 0: rows design[r] = (w M, w strain) for r in [off[t],
 // off[t+1]), eps[t] = lstsq's minimum-norm solution (NaN for other tasks).
+template <int LANES>
 __global__ __launch_bounds__(64) void k_pbp_strain_fit(const double* __restrict__ design,
                                                        const long long* __restrict__ off,
                                                        const int* __restrict__ worth, int T,
                                                        double* __restrict__ eps) {
-    const int t = (blockIdx.x * 64 + threadIdx.x) / GS_FIT_LANES;
-    const int sl = threadIdx.x & (GS_FIT_LANES - 1);
+    const int t = blockIdx.x * (64 / LANES) + threadIdx.x / LANES;
+    const int sl = threadIdx.x & (LANES - 1);
     const bool on = t < T && worth[t];
     double R[6][7];
 #pragma unroll
@@ -469,8 +475,8 @@ __global__ __launch_bounds__(64) void k_pbp_strain_fit(const double* __restrict_
 #pragma unroll
         for (int j = 0; j < 7; j++) R[i][j] = 0.0;
     const long long r0 = on ? off[t] : 0, r1 = on ? off[t + 1] : 0;
-    gs_qr_add_rows<6, 1, 2>(R, design, r0 + sl, r1, GS_FIT_LANES);
-    gs_qr_merge<6, 1>(R);  // every lane of the wave
+    gs_qr_add_rows<6, 1, LANES == 1 ? 4 : 2>(R, design, r0 + sl, r1, LANES);
+    gs_qr_merge<6, 1, LANES>(R);  // every lane of the wave
     if (t >= T || sl) return;
     double e[6];
     for (int i = 0; i < 6; i++) e[i] = __builtin_nan("");

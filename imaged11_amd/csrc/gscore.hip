@@ -1916,9 +1916,12 @@ int gs_pbp_merge_sums(const long long* perm, const long long* peak, long long np
     return GS_OK;
 }
 
-int gs_pbp_ubi_fit(const double* design, const long long* off, const int* fit,
-                   const double* ubi_in, const double B0[9], int T, double* ubifit, int* rank,
-                   int* worth, double* ubi_out, double* ub0, gs_stream_t stream) {
+// lanes per task where the number of rows is not known
+static int pbp_lanes(int T) { return T <= 1500 ? 16 : T <= 12288 ? 4 : 1; }
+
+int gs_pbp_ubi_fit_lanes(const double* design, const long long* off, const int* fit,
+                         const double* ubi_in, const double B0[9], int T, int lanes, double* ubifit,
+                         int* rank, int* worth, double* ubi_out, double* ub0, gs_stream_t stream) {
     DeviceCtx* ctx;
     GS_CHECK(get_ctx(&ctx));
     if (T < 0) return set_err(GS_ERR_ARG, "gs_pbp_ubi_fit: negative task count");
@@ -1926,22 +1929,44 @@ int gs_pbp_ubi_fit(const double* design, const long long* off, const int* fit,
     if (!B0) return set_err(GS_ERR_ARG, "gs_pbp_ubi_fit: null B0");
     gs_mat9 b;
     for (int i = 0; i < 9; i++) b.m[i] = B0[i];
-    hipLaunchKernelGGL(k_pbp_ubi_fit, dim3(blocks_for(T, 64 / GS_FIT_LANES)), dim3(64), 0, S(stream), design, off,
+    const auto kernel = lanes == 1    ? k_pbp_ubi_fit<1>
+                        : lanes == 4  ? k_pbp_ubi_fit<4>
+                        : lanes == 16 ? k_pbp_ubi_fit<16>
+                                      : nullptr;
+    if (!kernel) return set_err(GS_ERR_ARG, "gs_pbp_ubi_fit: %d lanes (1, 4 or 16)", lanes);
+    hipLaunchKernelGGL(kernel, dim3(blocks_for(T, 64 / lanes)), dim3(64), 0, S(stream), design, off,
                        fit, ubi_in, b, T, ubifit, rank, worth, ubi_out, ub0);
     GS_LAUNCHED();
     return GS_OK;
 }
 
-int gs_pbp_strain_fit(const double* design, const long long* off, const int* worth, int T,
-                      double* eps, gs_stream_t stream) {
+int gs_pbp_strain_fit_lanes(const double* design, const long long* off, const int* worth, int T,
+                            int lanes, double* eps, gs_stream_t stream) {
     DeviceCtx* ctx;
     GS_CHECK(get_ctx(&ctx));
     if (T < 0) return set_err(GS_ERR_ARG, "gs_pbp_strain_fit: negative task count");
     if (T == 0) return GS_OK;
-    hipLaunchKernelGGL(k_pbp_strain_fit, dim3(blocks_for(T, 64 / GS_FIT_LANES)), dim3(64), 0, S(stream), design,
-                       off, worth, T, eps);
+    const auto kernel = lanes == 1    ? k_pbp_strain_fit<1>
+                        : lanes == 4  ? k_pbp_strain_fit<4>
+                        : lanes == 16 ? k_pbp_strain_fit<16>
+                                      : nullptr;
+    if (!kernel) return set_err(GS_ERR_ARG, "gs_pbp_strain_fit: %d lanes (1, 4 or 16)", lanes);
+    hipLaunchKernelGGL(kernel, dim3(blocks_for(T, 64 / lanes)), dim3(64), 0, S(stream), design, off,
+                       worth, T, eps);
     GS_LAUNCHED();
     return GS_OK;
+}
+
+int gs_pbp_ubi_fit(const double* design, const long long* off, const int* fit,
+                   const double* ubi_in, const double B0[9], int T, double* ubifit, int* rank,
+                   int* worth, double* ubi_out, double* ub0, gs_stream_t stream) {
+    return gs_pbp_ubi_fit_lanes(design, off, fit, ubi_in, B0, T, pbp_lanes(T), ubifit, rank, worth,
+                                ubi_out, ub0, stream);
+}
+
+int gs_pbp_strain_fit(const double* design, const long long* off, const int* worth, int T,
+                      double* eps, gs_stream_t stream) {
+    return gs_pbp_strain_fit_lanes(design, off, worth, T, pbp_lanes(T), eps, stream);
 }
 
 int gs_pbp_rows_dot(const double* ubis, const long long* task, long long R, const double* g,

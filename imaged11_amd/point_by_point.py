@@ -18,7 +18,7 @@ Everything after the first selection works on the assigned rows only and
 is vectorised across all tasks at once on the device: the merge is one
 ordered segmented sum per column over (task, key) groups (the reference's
 per-voxel ``np.bincount``, the same sums in the same order), the
-least-squares fits run 16 lanes per task (``gs_pbp_ubi_fit``,
+least-squares fits run 1 to 16 lanes per task (``gs_pbp_ubi_fit``,
 ``gs_pbp_strain_fit``: the task's weighted rows streamed into QR factors by
 Givens rotations, merged, and decomposed by one-sided Jacobi rotations,
 then ``np.linalg.lstsq``'s minimum-norm solution, rank and rcond rule, and
@@ -319,13 +319,23 @@ def _score(ubis, task, g, tol):
     return hkl, ok
 
 
-def ubi_fit(design, off, fit, ubis, B0):
+def fit_lanes(T, rows):
+    """Lanes per task of the least-squares fits for T tasks with `rows` rows in
+    all: 1 where a task has few rows or the tasks fill the device, else 16
+    while those leave it idle, else 4 (the times are at k_pbp_ubi_fit)."""
+    if rows < 24 * T or T > 32768 or (T > 12288 and rows < 150 * T):
+        return 1
+    return 16 if T <= 1500 or (T <= 6000 and rows >= 120 * T) else 4
+
+
+def ubi_fit(design, off, fit, ubis, B0, lanes=None):
     """weighted_lstsq_ubi_fit (:408-419) and the fit-quality test
     (:1595-1597) of every task with fit[t], on the device
     (gs_pbp_ubi_fit): design (rows, 6) = (w g, w hkl) grouped by task with
     CSR offsets off (T+1).  Returns (ubifit, rank, worth, ubi_out, ub0):
     lstsq's solution and rank, the quality test, the fitted UBI where it
-    passes (else the input) and U.B0 of the fitted cell."""
+    passes (else the input) and U.B0 of the fitted cell.  lanes: of each
+    task, 1, 4 or 16 (fit_lanes chooses)."""
     lib = _lib.load()
     T = ubis.shape[0]
     dev = ubis.device
@@ -338,24 +348,26 @@ def ubi_fit(design, off, fit, ubis, B0):
     rank = torch.empty(T, dtype=torch.int32, device=dev)
     worth = torch.empty(T, dtype=torch.int32, device=dev)
     b0 = darr(np.asarray(B0, np.float64).reshape(9))
-    _lib.check(lib.gs_pbp_ubi_fit(dptr(design), dptr(off), dptr(fit_i), dptr(ubis), b0, T,
-                                  dptr(ubifit), dptr(rank), dptr(worth), dptr(ubi_out), dptr(ub0),
-                                  stream_ptr()), "pbp_ubi_fit")
+    lanes = lanes or fit_lanes(T, design.shape[0])
+    _lib.check(lib.gs_pbp_ubi_fit_lanes(dptr(design), dptr(off), dptr(fit_i), dptr(ubis), b0, T,
+                                        lanes, dptr(ubifit), dptr(rank), dptr(worth),
+                                        dptr(ubi_out), dptr(ub0), stream_ptr()), "pbp_ubi_fit")
     return ubifit, rank, worth.bool(), ubi_out, ub0
 
 
-def strain_fit(design, off, worth):
+def strain_fit(design, off, worth, lanes=None):
     """The strain lstsq of every task with worth[t] (:1652-1656) on the
     device (gs_pbp_strain_fit): design (rows, 7) = (w M, w strain) grouped
     by task.  Returns (T, 6) = (sxx, syy, szz, sxy, sxz, syz), NaN where
-    not fitted."""
+    not fitted.  lanes as for ubi_fit."""
     lib = _lib.load()
     T = worth.shape[0]
     w_i = worth.to(torch.int32).contiguous()
     design = design.contiguous()
     eps = torch.empty((T, 6), dtype=torch.float64, device=worth.device)
-    _lib.check(lib.gs_pbp_strain_fit(dptr(design), dptr(off), dptr(w_i), T, dptr(eps),
-                                     stream_ptr()), "pbp_strain_fit")
+    lanes = lanes or fit_lanes(T, design.shape[0])
+    _lib.check(lib.gs_pbp_strain_fit_lanes(dptr(design), dptr(off), dptr(w_i), T, lanes,
+                                           dptr(eps), stream_ptr()), "pbp_strain_fit")
     return eps
 
 

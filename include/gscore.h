@@ -476,7 +476,7 @@ int gs_pbp_merge_sums(const long long *perm, const long long *peak, long long np
                       const double *dty, const double *xpos, const double *eta,
                       const long long *goff, int G, double *out, gs_stream_t stream);
 
-/* The least-squares fits of refine_map, one thread per task t < T, as
+/* The least-squares fits of refine_map, some lanes per task t < T, as
  * np.linalg.lstsq solves them (minimum-norm solution, singular values of
  * the weighted design matrix <= eps * max(rows, columns) * the largest
  * taken as zero), rows of task t = [off[t], off[t+1]) of `design`:
@@ -496,6 +496,14 @@ int gs_pbp_ubi_fit(const double *design, const long long *off, const int *fit,
                    int *worth, double *ubi_out, double *ub0, gs_stream_t stream);
 int gs_pbp_strain_fit(const double *design, const long long *off, const int *worth, int T,
                       double *eps, gs_stream_t stream);
+/* The same with the given number of lanes per task (1, 4 or 16; the results
+ * differ in the rounding of the rows' order). */
+int gs_pbp_ubi_fit_lanes(const double *design, const long long *off, const int *fit,
+                         const double *ubi_in, const double B0[9], int T, int lanes,
+                         double *ubifit, int *rank, int *worth, double *ubi_out, double *ub0,
+                         gs_stream_t stream);
+int gs_pbp_strain_fit_lanes(const double *design, const long long *off, const int *worth, int T,
+                            int lanes, double *eps, gs_stream_t stream);
 
 /* Row products of refine_map's merged-peak scoring and strain fit
  * (ImageD11/sinograms/point_by_point.py:1581-1590,1611-1614,1639): per row
