@@ -150,6 +150,7 @@ SIEVE_TOL_MAX = 0.1  # the sieves pay while few of the pairs pass them
 
 LIST_SORT_MAX = 16384  # longest list gs_list_fill sorts
 ORDER_MAX = 8192       # most grains gs_list_order takes
+LIST_GRAINS_MAX = 65536  # most lists whose offsets one block should scan
 
 
 def score_mode(tol):

@@ -51,3 +51,19 @@ def test_order(dev, K):
     got = batched.list_order(torch.as_tensor(off, device=dev))
     assert got.dtype == torch.int32
     assert np.array_equal(got.cpu().numpy(), np.argsort(-length, kind="stable"))
+
+
+@pytest.mark.parametrize("n,K,pays", [(3000, _lib.LIST_GRAINS_MAX, True),
+                                      (3000, _lib.LIST_GRAINS_MAX + 1, False),
+                                      (_lib.LIST_SORT_MAX, 1, True),
+                                      (_lib.LIST_SORT_MAX + 1, 1, False)])
+def test_lists_at_the_limits(dev, n, K, pays):
+    assert batched.list_kernels_pay(K, n) == pays
+    rng = np.random.default_rng(n)
+    lab = rng.integers(-1, K, n).astype(np.int32)
+    lab[-1] = K - 1
+    idx, off, owner = (g.cpu().numpy() for g in batched.lists_from_labels(
+        torch.as_tensor(lab, device=dev), K))
+    order = np.argsort(np.where(lab < 0, K, lab), kind="stable")[:(lab >= 0).sum()]
+    assert np.array_equal(idx, order) and np.array_equal(owner, lab[order])
+    assert np.array_equal(off, np.searchsorted(lab[order], np.arange(K + 1)))
