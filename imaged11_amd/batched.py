@@ -313,7 +313,7 @@ def list_order(off):
     """Grain visiting order for the persistent refine: longest list first,
     equal lengths in grain order."""
     K = off.numel() - 1
-    if off.is_cuda and off.dtype == torch.int64 and off.is_contiguous() and 0 < K <= _lib.ORDER_MAX:
+    if _here(off) and off.dtype == torch.int64 and off.is_contiguous() and 0 < K <= _lib.ORDER_MAX:
         order = torch.empty(K, dtype=torch.int32, device=off.device)
         _lib.check(_ready().gs_list_order(dptr(off), K, dptr(order), stream_ptr()), "list_order")
         return order
@@ -420,8 +420,14 @@ def gv_assign_many(xl, so, co, wvln, ubis, trans, tol, drlv2, labels, grain_labe
     return out
 
 
+def _here(t):
+    """On the current device, whose stream the kernels take; another device's
+    tensor is torch's to handle."""
+    return t.is_cuda and t.device.index == torch.cuda.current_device()
+
+
 def _int32_labels(labels):
-    return (labels.is_cuda and labels.dtype == torch.int32 and labels.dim() == 1
+    return (_here(labels) and labels.dtype == torch.int32 and labels.dim() == 1
             and labels.is_contiguous() and labels.numel() < 2 ** 31)
 
 

@@ -1,7 +1,10 @@
 """The error bound of the matrix-core sieve, in numpy: h from f16 pieces,
 products exact, f32 accumulation that rounds or truncates at every step."""
+from types import SimpleNamespace
+
 import numpy as np
 import pytest
+import torch
 
 from imaged11_amd import batched
 
@@ -241,3 +244,13 @@ def test_the_score_takes_the_matrix_cores_where_they_were_measured_faster(K, pai
     for sign in (1, -1):
         assert batched.score_mfma_pays(K, N, sign * 0.02) == narrow
         assert batched.score_mfma_pays(K, N, sign * 0.05) == wide
+
+
+@pytest.mark.parametrize("index,current,ok", [(0, 0, True), (1, 0, False), (0, 1, False)])
+def test_labels_of_another_device_stay_with_torch(monkeypatch, index, current, ok):
+    """The list kernels launch on the current device's stream."""
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: current)
+    labels = SimpleNamespace(is_cuda=True, device=torch.device("cuda", index), dtype=torch.int32,
+                             dim=lambda: 1, is_contiguous=lambda: True, numel=lambda: 5)
+    assert batched._int32_labels(labels) == ok
+    assert not batched._int32_labels(torch.zeros(5, dtype=torch.int32))
