@@ -209,6 +209,16 @@ def orient_hits(uc, ring_1, ring_2, gv, hits, entries=None, with_cosines=False):
     return (ubis, cos) if with_cosines else ubis
 
 
+def sieve_pays(K, N, thr):
+    """Whether the lists are faster behind the matrix-core sieve.  Few pairs
+    pass at small thr; just above 0.01 (where tol^2 of tol = 0.1 rounds to)
+    the other kernel takes the slots of a wave with one atomic, which counts
+    when few grains own many peaks each: 8 x 2 10^6 6.2 ms against 14.4, 16 x
+    10^6 5.9 against 5.5."""
+    return (thr <= _lib.SIEVE_TOL_MAX ** 2 and batched.mfma_pays(K, N)
+            and (K >= 16 or thr <= 0.01))
+
+
 def select_lists(ubis, gv, thr, counts=None, sort=True):
     """CSR lists of the peaks each UBI indexes with the reference
     arithmetic (drlv2 < thr).  ubis (K,3,3) and gv (N,3) device tensors;
@@ -230,9 +240,8 @@ def select_lists(ubis, gv, thr, counts=None, sort=True):
     K, N = ubis.shape[0], gv.shape[0]
     cnt = torch.empty(K, dtype=torch.int32, device=dev)
 
-    # few pairs pass at small thr: the matrix-core sieve, where it pays
     ws = None
-    if thr <= _lib.SIEVE_TOL_MAX ** 2 and batched.mfma_pays(K, N):
+    if sieve_pays(K, N, thr):
         ws = _lib.sieve_ws(K, dev)
 
     def select(off, idx):

@@ -6,7 +6,7 @@ import numpy as np
 import pytest
 import torch
 
-from imaged11_amd import batched
+from imaged11_amd import batched, indexing
 
 
 def split16(v):
@@ -254,3 +254,10 @@ def test_labels_of_another_device_stay_with_torch(monkeypatch, index, current, o
                              dim=lambda: 1, is_contiguous=lambda: True, numel=lambda: 5)
     assert batched._int32_labels(labels) == ok
     assert not batched._int32_labels(torch.zeros(5, dtype=torch.int32))
+
+
+@pytest.mark.parametrize("K,N,thr,pays", [(8, 2000000, 0.01, True), (8, 2000000, 0.1 ** 2, False),
+                                          (16, 1000000, 0.1 ** 2, True), (16, 999999, 0.01, False),
+                                          (1000, 16000, 0.0101, False), (7, 10 ** 8, 0.01, False)])
+def test_selections_behind_the_sieve(K, N, thr, pays):
+    assert indexing.sieve_pays(K, N, thr) == pays
