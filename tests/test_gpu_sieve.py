@@ -485,3 +485,41 @@ def test_ball_dispatch(dev, K, N):
     for tol in (0.1, 0.11, 0.25, 0.74, 0.75):
         assert torch.equal(batched.score_many(ubi, gv, tol),
                            batched.score_many(ubi, gv, tol, mode=_lib.SCORE_CERTIFIED))
+
+
+# the kernels on the vector ALU: every call with labels of its own and every
+# tol > 0.1, over the ends of their LDS chunks (512 and 1024 grains)
+@pytest.mark.parametrize("K", [511, 512, 513, 1100])
+@pytest.mark.parametrize("own,tol", [(True, 0.05), (False, 0.2)])
+def test_scan_in_chunks_of_grains(dev, orc, K, own, tol):
+    N = 3000
+    ubi, trans, xl, so, co, w, rng = scan_inputs(K, N, K)
+    gl = rng.permutation(K + 50)[:K].astype(np.int32) if own else np.arange(K, dtype=np.int32)
+    d0, l0 = rng.uniform(0, 0.1, N), rng.integers(-2, K + 50, N).astype(np.int32)
+    d, lab = d0.copy(), l0.copy()
+    want = orc.gv_assign_many(xl, so, co, np.eye(3), w, ubi, trans, gl, tol, d, lab)
+    dd, ll = T(d0, dev), T(l0, dev, torch.int32)
+    got = batched.gv_assign_many(T(xl, dev), T(so, dev), T(co, dev), w, T(ubi, dev), T(trans, dev),
+                                 tol, dd, ll, grain_labels=T(gl, dev, torch.int32) if own else None,
+                                 mat=np.eye(3))
+    assert want.sum() > 0 and np.array_equal(got.cpu().numpy(), want)
+    assert np.array_equal(ll.cpu().numpy(), lab)
+    assert np.array_equal(dd.cpu().numpy().view(np.int64), d.view(np.int64))
+
+
+@pytest.mark.parametrize("K", [1023, 1024, 1025, 2100])
+@pytest.mark.parametrize("own,tol", [(True, 0.05), (False, 0.2)])
+def test_assignment_in_chunks_of_grains(dev, orc, K, own, tol):
+    N = 2500
+    ubi, gv = make(K, N, K)
+    rng = np.random.default_rng(K)
+    gl = rng.permutation(K + 50)[:K].astype(np.int32) if own else np.arange(K, dtype=np.int32)
+    d0, l0 = rng.uniform(0, 0.1, N), rng.integers(-2, K + 50, N).astype(np.int32)
+    d, lab = d0.copy(), l0.copy()
+    want = orc.assign_many(ubi, gl, gv, tol, d, lab)
+    dd, ll = T(d0, dev), T(l0, dev, torch.int32)
+    got = batched.assign_many(T(ubi, dev), T(gv, dev), tol, dd, ll,
+                              grain_labels=T(gl, dev, torch.int32) if own else None)
+    assert want.sum() > 0 and np.array_equal(got.cpu().numpy(), want)
+    assert np.array_equal(ll.cpu().numpy(), lab)
+    assert np.array_equal(dd.cpu().numpy().view(np.int64), d.view(np.int64))
