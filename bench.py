@@ -9,8 +9,9 @@ at 50 um / 150 mm, wavelength 0.2 A, omega 0-180 deg in 0.25 deg frames,
 timed region.  value = K*N*steps / elapsed.
 
 Printed: ONE JSON line, with a roofline object for the dominant kernel
-(k_score_mfma at tol <= 0.1, a sieve on the matrix cores; else
-k_score_many_fast, FP64 vector ALU bound) timed live with HIP events on its
+(k_score_mfma where batched.score_many takes the matrix cores, at the
+default sizes up to tol 0.75; else the row sieve or k_score_many_fast, FP64
+vector ALU bound) timed live with HIP events on its
 stream, and a cpu_baseline object: the reference C (oracle/_ref, compiled
 from its sources) running the same pipeline on the host cores, the grain
 loop spread over threads (ctypes releases the GIL), with its per-grain
@@ -36,7 +37,7 @@ ROOT = os.path.dirname(os.path.abspath(__file__))
 sys.path.insert(0, ROOT)
 
 FLOPS_PER_PAIR = 23      # h = UBI.g: 9 mul + 6 add; 3 sub; sumsq: 3 mul + 2 add
-# the matrix-core sieve (k_score_mfma, the default for tol <= 0.1): three
+# the matrix-core score (k_score_mfma: the sieve, beyond tol 0.1 the ball): three
 # v_mfma_f32_32x32x16_f16 for 32 peaks x 32 grains, i.e. 96 f16 flops per
 # pair executed (9 of the 16 k slots carry the split products)
 MFMA_FLOPS_PER_PAIR = 96
@@ -904,14 +905,19 @@ def main():
     score_ms = statistics.mean(a.elapsed_time(b) for a, b in evs)
     pairs = args.grains * args.peaks
     value = pairs * args.steps / (total_ms * 1e-3)
-    if (batched.score_mode(args.tol) == _lib.SCORE_SIEVE and
-            batched.score_mfma_pays(args.grains, args.peaks, args.tol)):
+    sieve = batched.score_mode(args.tol) == _lib.SCORE_SIEVE
+    if (batched.score_mfma_pays(args.grains, args.peaks, args.tol) if sieve
+            else batched.ball_pays(args.grains, args.peaks, args.tol)):
         kernel, bound, peak = "k_score_mfma", "mfma", PEAK_F16_MFMA
         achieved = MFMA_FLOPS_PER_PAIR * pairs / (score_ms * 1e-3)
-        frac_is = ("f16 matrix flops executed over the dense f16 peak; the kernel's vector "
-                   "instructions (3 per pair) run beside them, and the power limit bounds both")
+        frac_is = ("f16 matrix flops executed (96 per pair) over the dense f16 peak; the vector "
+                   "instructions beside them (%s) bound the kernel: at the default sizes the "
+                   "vector ALU is busy 82%% of the cycles, the matrix cores 25%%"
+                   % ("3.25 per pair in the sieve, 5.1 with queues and settling" if sieve
+                      else "11 per pair in the ball"))
     else:
-        kernel, bound, peak = "k_score_many_fast", "valu", PEAK_FP64_VALU
+        kernel = "k_score_many_sieve" if sieve else "k_score_many_fast"
+        bound, peak = "valu", PEAK_FP64_VALU
         achieved = FLOPS_PER_PAIR * pairs / (score_ms * 1e-3)
         frac_is = "algorithmic: flops_per_pair for every pair decided, over the FP64 peak"
     gpu_counts = counts.cpu().numpy()

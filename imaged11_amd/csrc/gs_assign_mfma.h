@@ -52,13 +52,14 @@
 // of one peak in one batch go through in lane order, which is grain order.
 //
 // Measured, labels, drlv2 and counts identical: 20 000 grains x 8 10^6 peaks
-// with positions 24.9 ms against 191 of k_gv_assign_many (FP64 VALU, 92%
+// with positions 23.9 ms against 191 of k_gv_assign_many (FP64 VALU, 92%
 // busy), 777 x 10^5 45 us against 310; g-vectors given, 500 x 200 003 36 us
-// against 230.  Per 32 x 32 tile: 51 vector instructions for the
-// sieve, 23 for pushes, settling and the tile's constants (the accumulator
-// start is rebuilt for each tile: kept across tiles in registers it made the
-// compiler copy and spill it, 37.7 ms), 421 cycles in all; bound, as the score,
-// by the power limit and what is left of latency at 3 waves per SIMD.
+// against 230.  Per 32 x 32 tile: 51 vector instructions for the sieve, 20 for
+// pushes, settling and the tile's constants (the accumulator start is rebuilt
+// for each tile: kept across tiles in registers it made the compiler copy and
+// spill it, 37.7 ms), 356 cycles in all.  Bound, as the score, by vector issue:
+// the vector ALU is busy 80% of the cycles and the matrix cores 27%, at 2.9
+// waves per SIMD and 2.2 GHz.
 #pragma once
 #include "gs_assign_gv.h"
 #include "gs_sieve.h"

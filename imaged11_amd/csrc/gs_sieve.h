@@ -8,13 +8,16 @@
 // pattern are then the fraction of h in units of 2^-16: no subtraction,
 // rounding or conversion is left for the vector ALU, which takes the maximum
 // of three 16-bit fields, the minimum over four pairs, and compares that:
-// three 16-bit instructions (2.4-2.8 cycles per wave each; v_max3_u16 and
-// v_min3_u16 take 8.4) and a quarter of a compare (4.2) per pair, against 11
-// FP64 instructions (4.5) of the row sieve k_score_many_sieve.  The MFMA's 32
-// cycles per 1024 products overlap them.  Measured, 1000 grains x 10^6 peaks,
-// tol 0.05: 146 us against 386; with the queue pushes off 120, with the
-// settling off 128.  What bounds it is the power limit: the same loop over
-// zeros runs a third faster than over data (201 against 270 cycles per tile).
+// three 16-bit instructions (2.4-2.8 cycles per wave each on their own;
+// v_max3_u16 and v_min3_u16 take 8.4) and a quarter of a compare (4.2) per pair,
+// 5.1 with the queues, the settling and the matrix instructions counted in,
+// against 11 FP64 instructions (4.5) of the row sieve k_score_many_sieve.  The
+// MFMA's 32 cycles per 1024 products overlap them.  Measured, 1000 grains x 10^6
+// peaks, tol 0.05: 146 us against 386; with the queue pushes off 120, with the
+// settling off 128.  Bound by vector issue: the vector ALU is busy 82% of the
+// cycles and the matrix cores 25%, at 2.4 GHz and 3.3 waves per SIMD; where no
+// pair passes, 88% of 24% fewer cycles, over constant data as over random
+// (292 000 and 296 000 against 383 000).
 //
 // Splitting.  u and g are each held as hi + lo in f16 (22 bits), and the
 // products hi hi + hi lo + lo hi use 9 of the 16 k slots:
@@ -39,9 +42,9 @@
 // counted.  The others (the cube of side 2r, 0.1% of random pairs at tol
 // 0.05, and the true hits) are settled one by one with the reference
 // arithmetic, so the sieve decides nothing that arithmetic would not.
-// A pair with a non-finite u or g has a NaN drlv2 and never counts: it may
-// pass or not, and is kept out of the bounds; peaks with one are given a
-// finite stand-in.  Larger A: up to GS_SIEVE_SPAN_WIDE the accumulator
+// A pair with a non-finite u or g has a NaN drlv2 and never counts: such peaks
+// and grains are kept out of the bounds and given a finite stand-in, in the
+// score the one that passes nothing (k_sieve_pack).  Larger A: up to GS_SIEVE_SPAN_WIDE the accumulator
 // starts at 1.5 2^27 (its last bit 2^-12 of h) and the fields are shifted
 // left by four first, error GS_SIEVE_ERR_WIDE = 2^-7 by the same count;
 // beyond that, and beyond |u| and |g|, the tile is tested in f32 on the
@@ -400,11 +403,12 @@ __device__ __forceinline__ gs_float16 gs_splat16(float v) {
 // Counters.  Atomics on one address from all over the chip go one after the
 // other, so the pairs are counted in private copies of the K counters, copy
 // blockIdx % copies for a block, which a last launch sums: a multiple of 8, so
-// that each copy is the business of one XCD, 8 to 64, up to 32768 counters in
-// all.  The assignment of 500 grains over 200 003 peaks took 112 us with one
-// copy and 36 with 64, the score of 24 x 10^6 31 us and 21, of 100 x 10^6 49
-// and 38; of 500 x 3 10^5 both took 43, and from there the score counts in
-// place (147 us against 152 at 1000 x 10^6, the sum's launch).
+// that each copy is the business of one XCD: 64 up to 512 grains, then 32768
+// counters in all, and from 2049 grains on 8.  The assignment of 500 grains
+// over 200 003 peaks took 112 us with one copy and 36 with 64, the score of
+// 24 x 10^6 31 us and 21, of 100 x 10^6 49 and 38; of 500 x 3 10^5 both took 43,
+// and from there the score counts in place (147 us against 152 at 1000 x 10^6,
+// the sum's launch).
 #define GS_SCORE_COPIES_MAX 256
 inline int gs_copies(int K) {
     const int c = 4096 / (K > 0 ? K : 1);

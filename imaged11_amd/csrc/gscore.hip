@@ -896,8 +896,8 @@ int score_and_assign(double ubi[3][3], double gv[][3], double tol, double* drlv2
     const size_t n = (size_t)ng;
     if (n * 36 <= GS_PINNED_MAX) {
         // as in score(): the peaks, drlv2 and labels stay in pinned memory,
-        // read once and written where they change.  Bound by the host's
-        // own copies: 20 000 peaks 139 us with five copies to the device and
+        // read once, drlv2 and labels written back once.  Bound by the
+        // host's own copies: 20 000 peaks 139 us with five copies to the device and
         // three back, 58 this way; 1500 100 and 30.
         std::vector<char*> h, d;
         if (pinned_slices({72, 4, 4, n * 24, n * 8, n * 4}, h, d) != GS_OK) return -1;
