@@ -442,20 +442,19 @@ def label_counts(labels, K):
     return torch.bincount(lab[(lab >= 0) & (lab < K)], minlength=K).to(torch.int32)
 
 
-def list_kernels_pay(K, n):
-    """Whether lists_from_labels of n labels and K grains goes through the list
-    kernels: their scan is one block's, with K = 10^6 3.7 ms against 0.37 of
-    torch's sort and scans, and with more peaks than the lists may hold
-    together one is surely (or by far most often) too long for the sort in
-    LDS, which costs the counting (1 x 10^5: 376 us against 332)."""
-    return 0 < K <= _lib.LIST_GRAINS_MAX and 0 < n <= K * _lib.LIST_SORT_MAX
+def list_kernels_pay(K):
+    """Whether lists_from_labels of K grains goes through the list kernels:
+    their scan is one block's, with K = 10^6 3.7 ms against 0.37 of torch's
+    sort and scans."""
+    return 0 < K <= _lib.LIST_GRAINS_MAX
 
 
 def lists_from_labels(labels, K):
     """CSR peak lists of grains 0..K-1 from per-peak labels (peaks in
     ascending order inside each list, label -1 and others dropped):
     returns (idx int32, off int64 (K+1,), owner int32)."""
-    if _int32_labels(labels) and list_kernels_pay(K, labels.numel()):
+    off = None
+    if _int32_labels(labels) and labels.numel() and list_kernels_pay(K):
         lib = _ready()
         dev, n = labels.device, labels.numel()
         counts = label_counts(labels, K)
@@ -471,16 +470,18 @@ def lists_from_labels(labels, K):
             _lib.check(lib.gs_list_fill(dptr(labels), n, K, dptr(off), dptr(cursor), longest,
                                         dptr(idx), dptr(owner), stream_ptr()), "list_fill")
             return idx, off, owner
+        # a list too long for the sort in LDS: the counts stay
     lab = labels.long()
     keep = (lab >= 0) & (lab < K)
     peaks = torch.nonzero(keep, as_tuple=False).flatten()
     order = torch.argsort(lab[peaks], stable=True)
     idx = peaks[order].to(torch.int32)
-    counts = torch.bincount(lab[peaks], minlength=K)
-    off = torch.zeros(K + 1, dtype=torch.int64, device=labels.device)
-    off[1:] = torch.cumsum(counts, 0)
+    if off is None:
+        counts, total = torch.bincount(lab[peaks], minlength=K), peaks.numel()
+        off = torch.zeros(K + 1, dtype=torch.int64, device=labels.device)
+        off[1:] = torch.cumsum(counts, 0)
     owner = torch.repeat_interleave(torch.arange(K, dtype=torch.int32, device=labels.device),
-                                    counts)
+                                    counts, output_size=total)
     return idx, off, owner
 
 

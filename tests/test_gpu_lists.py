@@ -53,17 +53,26 @@ def test_order(dev, K):
     assert np.array_equal(got.cpu().numpy(), np.argsort(-length, kind="stable"))
 
 
-@pytest.mark.parametrize("n,K,pays", [(3000, _lib.LIST_GRAINS_MAX, True),
-                                      (3000, _lib.LIST_GRAINS_MAX + 1, False),
-                                      (_lib.LIST_SORT_MAX, 1, True),
-                                      (_lib.LIST_SORT_MAX + 1, 1, False)])
-def test_lists_at_the_limits(dev, n, K, pays):
-    assert batched.list_kernels_pay(K, n) == pays
-    rng = np.random.default_rng(n)
-    lab = rng.integers(-1, K, n).astype(np.int32)
+@pytest.mark.parametrize("K", [_lib.LIST_GRAINS_MAX, _lib.LIST_GRAINS_MAX + 1])
+def test_lists_of_many_grains(dev, K):
+    assert batched.list_kernels_pay(K) == (K <= _lib.LIST_GRAINS_MAX)
+    rng = np.random.default_rng(K)
+    lab = rng.integers(-1, K, 3000).astype(np.int32)
     lab[-1] = K - 1
     idx, off, owner = (g.cpu().numpy() for g in batched.lists_from_labels(
         torch.as_tensor(lab, device=dev), K))
     order = np.argsort(np.where(lab < 0, K, lab), kind="stable")[:(lab >= 0).sum()]
     assert np.array_equal(idx, order) and np.array_equal(owner, lab[order])
     assert np.array_equal(off, np.searchsorted(lab[order], np.arange(K + 1)))
+
+
+def test_few_of_many_labels_stay_with_the_kernels(dev, monkeypatch):
+    """Short lists among a great many peaks of no grain."""
+    n, K = 8 * _lib.LIST_SORT_MAX, 2
+    lab = np.full(n, -1, np.int32)
+    lab[5::1000] = np.arange(len(lab[5::1000])) % K
+    t = torch.as_tensor(lab, device=dev)
+    monkeypatch.setattr(torch, "nonzero", None)  # torch's route
+    got = batched.lists_from_labels(t, K)
+    for g, w in zip(got, reference(lab, K)):
+        assert np.array_equal(g.cpu().numpy(), w)
