@@ -81,7 +81,7 @@ __device__ __forceinline__ float gs_uniform(float v) {
 
 // Fragments and tile_info of every tile, the exponent y, the counters cleared.
 // xl (GEOM): the ng peaks, ds = 1/wavelength; y is every block's own, from the
-// median |xl| of the same 128 of them.
+// median |xl| of the same 64 of them.
 template <bool GEOM>
 __global__ __launch_bounds__(128) void k_assign_pack(const double* __restrict__ ubis,
                                                      const double* __restrict__ trans, int K,
@@ -91,26 +91,40 @@ __global__ __launch_bounds__(128) void k_assign_pack(const double* __restrict__ 
                                                      gs_tile_info* __restrict__ info,
                                                      int* __restrict__ yexp,
                                                      int* __restrict__ priv, int copies) {
-    __shared__ float lspan[128], llin[128], lt[128];
+    __shared__ __align__(16) float lspan[128], llin[128], lt[128];
     const int tl = blockIdx.x, t = threadIdx.x;
+    const int row = t / 32, col = t & 31;
+    const int g = min(32 * tl + col, K - 1);
+    // everything that is read, on its way at once
+    const double* u = ubis + 9 * (size_t)g + 3 * min(row, 2);
+    double u0 = u[0], u1 = u[1], u2 = u[2], t0 = 0.0, t1 = 0.0, t2 = 0.0;
+    float n2 = __builtin_inff();  // |xl|^2 of the thread's sample
+    if constexpr (GEOM) {
+        t0 = trans[3 * (size_t)g];
+        t1 = trans[3 * (size_t)g + 1];
+        t2 = trans[3 * (size_t)g + 2];
+        const double* x = xl + 3 * ((long long)(t & 63) * ng / 64);
+        const float s = (float)(x[0] * x[0] + x[1] * x[1] + x[2] * x[2]);
+        n2 = s > 0.0f ? s : n2;  // NaN: not one either
+    }
     if (32 * tl + (t & 31) < K)
         for (int c = t / 32; c < copies; c += 4) priv[(size_t)c * K + 32 * tl + (t & 31)] = 0;
     int y = 0;
     if constexpr (GEOM) {
-        const double* x = xl + 3 * ((long long)t * ng / 128);
-        const double n2 = x[0] * x[0] + x[1] * x[1] + x[2] * x[2];
-        const float len = n2 > 0.0 ? (float)sqrt(n2) : __builtin_inff();  // NaN: not one either
-        lt[t] = len;
+        if (t < 64) lt[t] = n2;
         if (t == 0) lspan[0] = __builtin_inff();
         __syncthreads();
-        int rank = 0, n = 0;
-        for (int i = 0; i < 128; i++) {
-            rank += lt[i] < len || (lt[i] == len && i < t);
-            n += lt[i] < __builtin_inff();
+        if (t < 64) {
+            int rank = 0, n = 0;
+#pragma unroll
+            for (int i = 0; i < 64; i++) {
+                rank += lt[i] < n2 || (lt[i] == n2 && i < t);
+                n += lt[i] < __builtin_inff();
+            }
+            if (rank == n / 2) lspan[0] = n2;
         }
-        if (rank == n / 2) lspan[0] = len;
         __syncthreads();
-        const float r = 64.0f * fabsf((float)ds) / lspan[0];
+        const float r = 64.0f * fabsf((float)ds) / sqrtf(lspan[0]);
         int e = 0;
         if (r > 0.0f && r < __builtin_inff()) (void)frexpf(r, &e);
         y = max(-60, min(60, e - 1));
@@ -119,15 +133,6 @@ __global__ __launch_bounds__(128) void k_assign_pack(const double* __restrict__ 
     }
     lspan[t] = llin[t] = lt[t] = 0.0f;
     if (t < 96) {  // one grain row each
-        const int row = t / 32, col = t & 31;
-        const int g = min(32 * tl + col, K - 1);
-        const double* u = ubis + 9 * (size_t)g + 3 * row;
-        double u0 = u[0], u1 = u[1], u2 = u[2], t0 = 0.0, t1 = 0.0, t2 = 0.0;
-        if constexpr (GEOM) {
-            t0 = trans[3 * (size_t)g];
-            t1 = trans[3 * (size_t)g + 1];
-            t2 = trans[3 * (size_t)g + 2];
-        }
         float a = (float)(fabs(u0) + fabs(u1) + fabs(u2));
         const float at = (float)(fabs(t0) + fabs(t1) + fabs(t2));
         if (!(a < __builtin_inff() && at < __builtin_inff())) {
@@ -151,14 +156,16 @@ __global__ __launch_bounds__(128) void k_assign_pack(const double* __restrict__ 
         f[col + 32] = hi;
     }
     __syncthreads();
-    if (t == 0) {
-        gs_tile_info w = {0.0f, 0.0f, 0.0f, 0.0f};
-        for (int i = 0; i < 96; i++) {
-            w.span = fmaxf(w.span, lspan[i]);
-            w.lin = fmaxf(w.lin, llin[i]);
-            w.tmax = fmaxf(w.tmax, lt[i]);
+    if (t < 32) {
+        gs_tile_info w = {fmaxf(lspan[t], fmaxf(lspan[t + 32], lspan[t + 64])),
+                          fmaxf(llin[t], fmaxf(llin[t + 32], llin[t + 64])),
+                          fmaxf(lt[t], fmaxf(lt[t + 32], lt[t + 64])), 0.0f};
+        for (int o = 16; o > 0; o >>= 1) {
+            w.span = fmaxf(w.span, __shfl_xor(w.span, o, 32));
+            w.lin = fmaxf(w.lin, __shfl_xor(w.lin, o, 32));
+            w.tmax = fmaxf(w.tmax, __shfl_xor(w.tmax, o, 32));
         }
-        info[tl] = w;
+        if (t == 0) info[tl] = w;
     }
 }
 
